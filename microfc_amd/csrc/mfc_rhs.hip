@@ -65,6 +65,11 @@ constexpr int kBaseOnZ = 4;
 // inside the contracted form's 1e-12.  The plain FP64 form keeps the
 // per-cell coefficients unless they are equal bit for bit.
 constexpr double kUniformRelTol = 5e-13;
+// WENO5 coefficients of cells of equal width (plane order of mfc_device.hpp).
+constexpr double kCanon[kNCoef] = {
+    1.0 / 3, -5.0 / 6, -1.0 / 6, -1.0 / 3, -2.0 / 3, 1.0 / 6, -1.0 / 6, 2.0 / 3,   1.0 / 3,
+    1.0 / 6, 5.0 / 6,  -1.0 / 3, 0.1,      0.6,      0.3,     0.3,      0.6,       0.1,
+    4.0 / 3, -11.0 / 3, 10.0 / 3, 4.0 / 3, -5.0 / 3, 4.0 / 3, 10.0 / 3, -11.0 / 3, 4.0 / 3};
 // The fused x and y sweep, and the RK-base variables the z sweep adds before
 // it (512^3: 47.7, 46.0, 44.9, 44.8, 45.9 ms per step with 0, 2, 4, 6, 8 of
 // the 8; the fused sweep is bound by VALU issue, the z sweep less so; FP32
@@ -1089,6 +1094,12 @@ int mfc_rhs_set_grid(int dir, const double *s_cb, const double *ds) {
             }
         }
     }
+    // The contracted form's uniform-grid WENO5 kernels have the constants of
+    // equal cell widths built in (weno5_canon): equal coefficients of unequal
+    // widths (a geometric grid) run the per-cell kernels.
+    if (G.prm.precision == MFC_PREC_FP64_FAST && G.prm.weno_order == 5)
+        for (int q = 0; q < kNCoef && D.uniform; ++q)
+            D.uniform = std::fabs(D.ucf[q] - kCanon[q]) <= kUniformRelTol * std::fabs(kCanon[q]);
     // ... and over every cell with coefficients (the weno_Re_flux gradient
     // pass reconstructs the ghost cells too)
     {

@@ -691,7 +691,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(ML ? 2 : 4, 
             R st[WO], vl, vr;
 #pragma unroll
             for (int w = 0; w < WO; ++w) st[w] = sp[v][lane + w];
-            weno_cell<WO, R, true, true>(st, cf, eps, vl, vr);
+            weno_both<WO, R, UNI>(st, cf, eps, vl, vr, CanonK());
             const R vn = __shfl_down(vl, 1, 64);
             sp[v][lane] = vr;
             sp[v][64 + lane] = vn;
@@ -1117,7 +1117,7 @@ __global__ __launch_bounds__((tc_cols<R, ML>(DIR) * tc_rows<R>(DIR)))
             R st[WO], vl;
 #pragma unroll
             for (int w = 0; w < WO; ++w) st[w] = sp[v][tx][ts + w];
-            weno_cell<WO, R, true, true>(st, cf, eps, vl, qL[v]);
+            weno_both<WO, R, UNI>(st, cf, eps, vl, qL[v], CanonK());
             qR[v] = row_next<kTS>(vl);
         }
     }
@@ -1297,7 +1297,7 @@ __global__ __launch_bounds__(kXyThreads) __attribute__((amdgpu_waves_per_eu(4, 8
             R st[5], vl;
 #pragma unroll
             for (int w = 0; w < 5; ++w) st[w] = sp[v][cx][yr + w];
-            weno_cell<5, R, true, true>(st, cf, eps, vl, qL[v]);
+            weno_both<5, R, true>(st, cf, eps, vl, qL[v], CanonK());
             qR[v] = __shfl_down(vl, 1u, YK);
         }
         const int jf = y0 - 1 + yr;
@@ -1325,7 +1325,7 @@ __global__ __launch_bounds__(kXyThreads) __attribute__((amdgpu_waves_per_eu(4, 8
             R st[5], vl;
 #pragma unroll
             for (int w = 0; w < 5; ++w) st[w] = sp[v][c + w][ry];
-            weno_cell<5, R, true, true>(st, cf, eps, vl, qL[v]);
+            weno_both<5, R, true>(st, cf, eps, vl, qL[v], CanonK());
             qR[v] = __shfl_down(vl, 1u, XL);
         }
         const int jf = x0 - 1 + c;
