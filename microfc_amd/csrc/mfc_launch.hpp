@@ -3,12 +3,13 @@
 // launch_sweep<N> so the kernel variants compile in parallel.
 #pragma once
 
+#include "mfc_march.hpp"
 #include "mfc_sweep.hpp"
 
 namespace mfc {
 
 struct SweepLaunch {
-    int dir;       // 0, 1, 2; 3: the fused x and y sweep (k_sweep_xy)
+    int dir;       // 0, 1, 2; 3: the fused x and y sweep (k_sweep_xy); 4: the x and y march; 5: the z march
     int num_dims;  // 1..3
     int weno_order;
     int precision; // MFC_PREC_*
@@ -25,7 +26,13 @@ int launch_sweep(const SweepLaunch &L, const SweepArgs &a, hipStream_t st);
     template <int D, int WO, typename R, bool ML, bool UNI>                                             \
     static int launch_nf##NF##_dwrm(int dir, const SweepArgs &a, hipStream_t st) {                      \
         const dim3 grid((unsigned)a.nblocks);                                                           \
-        if (dir == 3) {                                                                                 \
+        if (dir == 4) {                                                                                 \
+            if constexpr (NF <= kMarchMaxFluids && D >= 2 && WO == 5 && !ML && (sizeof(R) == 8 || !UNI)) hipLaunchKernelGGL((k_march<NF, D, 1, R, true, UNI>), grid, dim3(64), 0, st, a); \
+            else return -1;                                                                             \
+        } else if (dir == 5) {                                                                          \
+            if constexpr (NF <= kMarchMaxFluids && D == 3 && WO == 5 && !ML) hipLaunchKernelGGL((k_march<NF, 3, 2, R, false, UNI>), grid, dim3(64), 0, st, a); \
+            else return -1;                                                                             \
+        } else if (dir == 3) {                                                                          \
             if constexpr (NF <= kXyMaxFluids && D >= 2 && WO == 5 && !ML && UNI) hipLaunchKernelGGL((k_sweep_xy<NF, D, R>), grid, dim3(kXyThreads), 0, st, a); \
             else return -1;                                                                             \
         } else if (dir == 0) {                                                                          \

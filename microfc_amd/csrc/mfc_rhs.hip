@@ -70,12 +70,26 @@ constexpr double kCanon[kNCoef] = {
     1.0 / 3, -5.0 / 6, -1.0 / 6, -1.0 / 3, -2.0 / 3, 1.0 / 6, -1.0 / 6, 2.0 / 3,   1.0 / 3,
     1.0 / 6, 5.0 / 6,  -1.0 / 3, 0.1,      0.6,      0.3,     0.3,      0.6,       0.1,
     4.0 / 3, -11.0 / 3, 10.0 / 3, 4.0 / 3, -5.0 / 3, 4.0 / 3, 10.0 / 3, -11.0 / 3, 4.0 / 3};
-// The fused x and y sweep, and the RK-base variables the z sweep adds before
-// it (512^3: 47.7, 46.0, 44.9, 44.8, 45.9 ms per step with 0, 2, 4, 6, 8 of
-// the 8; the fused sweep is bound by VALU issue, the z sweep less so; FP32
-// bulk the same way: 42.4, 41.0, 40.8, 41.3 ms with 2, 4, 6, 8).
 constexpr bool kFuseXY = true;
-constexpr int kBaseOnZFused = 6;
+// Waves of a march the chip runs at a time (8 per CU), and the fewest rows of
+// a chunk.
+constexpr int kMarchSlots = 8 * 256, kMarchRowsMin = 16;
+// Cells from which a march (k_march) takes over, where both were measured
+// (ms per RK3 step, tile kernels -> marches; two fluids):
+//  * equal widths, 3D: contracted FP64 128^3 0.82 -> 0.82, 200^3 2.72 -> 2.63,
+//    512^3 42.1 -> 36.8; plain FP64 128^3 1.45 -> 1.43; one RHS at 256^3
+//    3.52 -> 3.24;
+//  * equal widths, 2D: contracted 2048^2 0.73 -> 0.79, 4096^2 2.70 -> 2.54;
+//    plain 2048^2 1.36 -> 1.50, 4096^2 5.13 -> 5.02;
+//  * other widths, against the separate sweeps: contracted 1024^2 0.326 ->
+//    0.331, 1500^2 0.78 -> 0.52, 4096^2 5.53 -> 3.10, 96^3 0.51 -> 0.48, 128^3
+//    1.36 -> 0.93, 200^3 4.95 -> 2.97; plain 1024^2 0.49 -> 0.56, 1500^2 1.02 ->
+//    0.92, 4096^2 7.41 -> 5.74, 96^3 0.77 -> 0.79, 200^3 6.74 -> 4.93; FP32 bulk
+//    1024^2 0.26 -> 0.29, 2048^2 1.22 -> 0.86, 96^3 0.41 -> 0.48, 200^3 4.10 ->
+//    3.33.
+// The FP32-bulk form on equal widths keeps its tiles (300 x 250 x 200 4.75 ->
+// 4.91): with half the LDS and registers they fill the SIMDs already.
+constexpr double kMarchUniform2D = 8e6, kMarchUniform3D = 3e6, kMarchPerCell = 1.5e6;
 
 thread_local std::string g_err;
 
@@ -765,14 +779,62 @@ SweepArgs xy_args() {
     return a;
 }
 
-// d = 0, 1, 2: one direction; d = 3: the fused x and y sweep.
+// Arguments of a march (k_march): d = 4 the y march with the x faces, d = 5
+// the z march.
+SweepArgs march_args(int d) {
+    SweepArgs a = d == 4 ? xy_args() : sweep_args(2);
+    const int cells = d == 4 ? kMarchCellsXY : kMarchCellsZ, rows = d == 4 ? G.prm.n + 1 : G.prm.p + 1;
+    const int other = d == 4 ? G.prm.p + 1 : G.prm.n + 1;
+    if (d == 4) {
+        a.coef2 = G.dir[1].coef;
+        a.ncell2 = G.dir[1].s + 2 * G.b + 1;
+        a.uniform = G.dir[0].uniform && G.dir[1].uniform;
+    }
+    a.rl = d == 4 ? G.prm.m + 1 + 2 * kMarchHaloXY : G.prm.m + 1;
+    a.ntile = (int)(((long)a.rl * other + cells - 1) / cells);
+    // Chunks of rows: a chunk costs three rows more than it finishes (the
+    // staged rows and the reconstructions before its first face), and the
+    // chip runs kMarchSlots waves at a time, the last round half empty.
+    double best = 0.0;
+    for (int nc = 1; nc <= rows; ++nc) {
+        const int L = (rows + nc - 1) / nc;
+        if (L < kMarchRowsMin && nc > 1) break;
+        if ((rows + L - 1) / L != nc) continue;
+        const double rounds = std::max(1.0, (double)a.ntile * nc / kMarchSlots + 0.5);
+        const double cost = rounds * (L + 3);
+        if (best == 0.0 || cost < best) best = cost, a.chunk = L, a.nchunk = nc;
+    }
+    a.nblocks = (long)a.ntile * a.nchunk;
+    return a;
+}
+
+// Whether the x and y directions (d = 4) or the z direction (d = 5) of a
+// WENO5 case of the plain, contracted or FP32-bulk form run as a march.
+bool marches(int d) {
+    if (G.visc || G.prm.precision == MFC_PREC_FP32_LEARNED || G.prm.weno_order != 5 ||
+        G.prm.num_fluids > kMarchMaxFluids || G.D < (d == 4 ? 2 : 3))
+        return false;
+    if (G.ng * (long)sizeof(double) >= (1L << 32)) return false; // 32-bit byte offsets within a variable
+    const bool uni = d == 4 ? G.dir[0].uniform && G.dir[1].uniform : G.dir[2].uniform;
+    if (uni && G.prm.precision == MFC_PREC_FP32_BULK) return false;
+    if ((double)G.nint < (!uni ? kMarchPerCell : G.D == 2 ? kMarchUniform2D : kMarchUniform3D)) return false;
+    // short rows or few of them: the lanes and rows a march adds at the ends
+    // would outweigh what it saves
+    const SweepArgs a = march_args(d);
+    return a.chunk >= kMarchRowsMin &&
+           (double)G.nint / (d == 4 ? G.prm.n + 1 : G.prm.p + 1) >=
+               0.85 * a.ntile * (d == 4 ? kMarchCellsXY : kMarchCellsZ);
+}
+
+// d = 0, 1, 2: one direction; d = 3: the fused x and y sweep; d = 4, 5: the
+// marches.
 int sweep(int d, SweepArgs &a) {
     SweepLaunch L{d, G.D, G.prm.weno_order, G.prm.precision};
     if (G.prm.precision == MFC_PREC_FP32_LEARNED) {
         a.mlp = mlp_frags();
         if (!a.mlp) return fail(-4, "learned weights requested but mfc_mlp_init has not been called");
     }
-    TimedScope ts(d == 3 ? kKSweepXY : kKSweepX + d);
+    TimedScope ts(d == 3 || d == 4 ? kKSweepXY : d == 5 ? kKSweepZ : kKSweepX + d);
     int rc;
     const int form = G.prm.precision == MFC_PREC_FP64        ? kFormF64
                      : G.prm.precision == MFC_PREC_FP64_FAST ? kFormF64Fast
@@ -900,15 +962,16 @@ int sweeps(const Fields &qin, const Fields &rhs, int rk, const Fields *qbase, co
         ci += cb;
         cb = 0.0;
     }
-    // The contracted and FP32-bulk forms on grids uniform in x and y, WENO5,
-    // one or two fluids, fuse the y and x sweeps (k_sweep_xy): in 3D after
-    // the z sweep, in 2D alone.
+    // The contracted and FP32-bulk forms, WENO5, one or two fluids, fuse the y
+    // and x sweeps on grids uniform in x and y (k_sweep_xy) or large enough for
+    // a march (k_march): in 3D after the z sweep, in 2D alone.
+    const bool march = marches(4), marchz = marches(5);
     const bool fuse = reverse && kFuseXY && G.D >= 2 &&
                       (G.prm.precision == MFC_PREC_FP64_FAST || G.prm.precision == MFC_PREC_FP32_BULK) &&
-                      G.prm.weno_order == 5 && G.prm.num_fluids <= kXyMaxFluids && G.dir[0].uniform &&
-                      G.dir[1].uniform;
+                      G.prm.weno_order == 5 && G.prm.num_fluids <= kXyMaxFluids &&
+                      (march || (G.dir[0].uniform && G.dir[1].uniform));
     if (fuse) {
-        const int split = G.D == 3 ? kBaseOnZFused : 0;
+        const int split = G.D == 3 ? std::min(kBaseOnZFused, G.S) : 0;
         auto stage = [&](SweepArgs &a, int fold_kind, int lo, int hi) {
             a.qin = qin;
             a.rhs = rhs;
@@ -926,22 +989,22 @@ int sweeps(const Fields &qin, const Fields &rhs, int rk, const Fields *qbase, co
             }
         };
         if (G.D == 3) {
-            SweepArgs a = sweep_args(2);
+            SweepArgs a = marchz ? march_args(5) : sweep_args(2);
             stage(a, 1, 0, split);
             a.accumulate = 0;
-            if (int rc = sweep(2, a)) return rc;
+            if (int rc = sweep(marchz ? 5 : 2, a)) return rc;
         }
-        SweepArgs a = xy_args();
+        SweepArgs a = march ? march_args(4) : xy_args();
         stage(a, 3, split, G.S);
         a.accumulate = G.D == 3;
-        return sweep(3, a);
+        return sweep(march ? 4 : 3, a);
     }
     // The plain form fuses its first two directions the same way (bitwise
     // the separate x and y sweeps): in 3D the z sweep then adds its part and
     // applies the RK stage, in 2D the fused sweep applies it.
     const bool fuse_plain = kFuseXY && !G.visc && G.D >= 2 && G.prm.precision == MFC_PREC_FP64 &&
-                            G.prm.weno_order == 5 && G.prm.num_fluids <= kXyMaxFluids && G.dir[0].uniform &&
-                            G.dir[1].uniform;
+                            G.prm.weno_order == 5 && G.prm.num_fluids <= kXyMaxFluids &&
+                            (march || (G.dir[0].uniform && G.dir[1].uniform));
     if (fuse_plain) {
         auto finish = [&](SweepArgs &a, bool last) {
             a.qin = qin;
@@ -954,15 +1017,15 @@ int sweeps(const Fields &qin, const Fields &rhs, int rk, const Fields *qbase, co
                 a.base_is_in = qbase->v[0] == qin.v[0];
             }
         };
-        SweepArgs a = xy_args();
+        SweepArgs a = march ? march_args(4) : xy_args();
         finish(a, G.D == 2);
         a.accumulate = 0;
-        if (int rc = sweep(3, a)) return rc;
+        if (int rc = sweep(march ? 4 : 3, a)) return rc;
         if (G.D == 3) {
-            SweepArgs z = sweep_args(2);
+            SweepArgs z = marchz ? march_args(5) : sweep_args(2);
             finish(z, true);
             z.accumulate = 1;
-            return sweep(2, z);
+            return sweep(marchz ? 5 : 2, z);
         }
         return 0;
     }

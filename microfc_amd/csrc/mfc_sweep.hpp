@@ -86,7 +86,19 @@ struct SweepArgs {
     int bc2_beg, bc2_end;
     double ucf2[kNCoef];
     float ucf2_32[kNCoef];
+    // k_march with the x faces: the y direction's coefficient table
+    const double *coef2;
+    long ncell2;
+    int rl; // entries per row of the outer index (k_march)
 };
+
+// RK-base variables the z sweep adds before the fused x and y sweep
+// (512^3: 47.7, 46.0, 44.9, 44.8, 45.9 ms per step with 0, 2, 4, 6, 8 of
+// the 8; the fused sweep is bound by VALU issue, the z sweep less so; FP32
+// bulk the same way: 42.4, 41.0, 40.8, 41.3 ms with 2, 4, 6, 8).
+constexpr int kBaseOnZFused = 6;
+// Column sets that take all their chunks before the next sets (k_march).
+constexpr int kMarchGroup = 64;
 
 // Threads per column of the cell-parallel y/z tile by form.  Measured on
 // MI355X: in the plain FP64 form 32 (512-thread blocks, 30 cells per column)
@@ -306,7 +318,7 @@ __device__ __forceinline__ void rk_combine(const SweepArgs &a, const FinishIn<S>
 template <int NF, int D, typename R, int M, typename O>
 __device__ __forceinline__ void finish_cell(const SweepArgs &a, O go, O ro, double inv,
                                             const R *Fm, const R *Fp, R usm, R usp,
-                                            const FinishIn<Sys<NF, D>::S> &f) {
+                                            const FinishIn<Sys<NF, D>::S> &f, int lo, int hi) {
     using Y = Sys<NF, D>;
     constexpr int S = Y::S;
     double r[S];
@@ -324,7 +336,7 @@ __device__ __forceinline__ void finish_cell(const SweepArgs &a, O go, O ro, doub
                     // pressure, dF is a cancellation whose separate
                     // rounding doubled the error against the oracle
                     double acc = a.fold == 1 ? 0.0 : f.rhs[v];
-                    if (v >= a.base_lo && v < a.base_hi) acc = fma(a.cb, f.base[v], acc);
+                    if (a.cb != 0.0 && v >= lo && v < hi) acc = fma(a.cb, f.base[v], acc);
                     r[v] = fma(sc, df, acc);
                 } else
                     r[v] = f.rhs[v] + sc * df;
@@ -740,7 +752,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(ML ? 2 : 4, 
             const Off go{ghost_off(a, x0, j, k), (unsigned)lane}, ro{interior_off(a, x0, j, k), (unsigned)lane};
             FinishIn<S> fin;
             finish_load_staged<NF, D, FM>(a, go, ro, cin, 1, fin);
-            finish_cell<NF, D, R, FM>(a, go, ro, a.inv_ds[i], f, fp, us, usp, fin);
+            finish_cell<NF, D, R, FM>(a, go, ro, a.inv_ds[i], f, fp, us, usp, fin, a.base_lo, a.base_hi);
         }
         return;
     }
@@ -776,7 +788,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(ML ? 2 : 4, 
             finish_load_staged<NF, D, FM>(a, go, ro, cin, 1, fin);
         else
             finish_load<NF, D, FM>(a, go, ro, fin);
-        finish_cell<NF, D, R, FM>(a, go, ro, a.inv_ds[i], Fm, Fp, sf[S][lane], sf[S][lane + 1], fin);
+        finish_cell<NF, D, R, FM>(a, go, ro, a.inv_ds[i], Fm, Fp, sf[S][lane], sf[S][lane + 1], fin, a.base_lo, a.base_hi);
     }
 }
 
@@ -965,7 +977,7 @@ __global__ __launch_bounds__(t_threads<ML>()) __attribute__((amdgpu_waves_per_eu
         else
             finish_load<NF, D, FM>(a, gcell(i, cc), rcell(i, cc), fin);
         finish_cell<NF, D, R, FM>(a, gcell(i, cc), rcell(i, cc), a.inv_ds[cc], Fm, Fp, sf[S][ts][tx],
-                                  sf[S][ts + 1][tx], fin);
+                                  sf[S][ts + 1][tx], fin, a.base_lo, a.base_hi);
     }
 }
 
@@ -1162,7 +1174,92 @@ __global__ __launch_bounds__((tc_cols<R, ML>(DIR) * tc_rows<R>(DIR)))
             finish_load_staged<NF, D, FM>(a, go, ro, &lcons[0][fx][fs], XC * KP, fin);
         else
             finish_load<NF, D, FM>(a, go, ro, fin);
-        finish_cell<NF, D, R, FM>(a, go, ro, a.inv_ds[cc], Fm, Fp, fl[S][fs][fx], fl[S][fs + 1][fx], fin);
+        finish_cell<NF, D, R, FM>(a, go, ro, a.inv_ds[cc], Fm, Fp, fl[S][fs][fx], fl[S][fs + 1][fx], fin, a.base_lo, a.base_hi);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// The part of a cell's finish of x and y that comes before x: rhs (z's part in
+// 3D), the RK base in a spread stage, the y divergence; in the plain form,
+// which adds x first, the y difference itself.  fold: a.fold; sy: the y
+// difference's factor; rhs(), base(): the operands; with_base: whether this
+// sweep adds this variable's base.
+template <typename R, typename LR, typename LB>
+__device__ __forceinline__ double finish_y_part(const SweepArgs &a, bool fold, double sy, double dfy, bool with_base,
+                                                LR &&rhs, LB &&base) {
+    if constexpr (!kFastF64 && sizeof(R) == 8) {
+        return dfy;
+    } else {
+        double acc = a.accumulate ? rhs() : 0.0;
+        if (fold && a.cb != 0.0 && with_base) acc = __builtin_fma(a.cb, base(), acc);
+        return __builtin_fma(sy, dfy, acc);
+    }
+}
+
+// Finish of a cell's x and y directions together from its flux differences
+// (dfx, y_part(v, fold, sy): finish_y_part; lower minus upper flux, in FP64;
+// the FP32-bulk form converts its fluxes) and contact-velocity differences,
+// with the stage input and the plain form's RK base in f: the divergence, the
+// alpha*div(u) sources and the rhs store or the RK stage (out: where the
+// output pointers are read from).
+template <int NF, int D, typename R, typename O, typename YP>
+__device__ __forceinline__ void finish_xy(const SweepArgs &a, const SweepArgs &out, O go, O ro, double ix, double iy,
+                                          const double *dfx, double dusx, double dusy,
+                                          const FinishIn<Sys<NF, D>::S> &f, YP &&y_part) {
+    using Y = Sys<NF, D>;
+    constexpr int S = Y::S;
+    double r[S];
+    if constexpr (!kFastF64 && sizeof(R) == 8) {
+        // plain FP64: the x sweep's finish (the first direction: it assigns)
+        // and then the y sweep's, operation for operation, so the result is
+        // bitwise theirs; then the rhs store or the RK stage (2D, where y is
+        // the last direction)
+#pragma unroll
+        for (int v = 0; v < S; ++v) r[v] = ix * dfx[v];
+#pragma unroll
+        for (int q = 0; q < NF; ++q) r[Y::ADV + q] = r[Y::ADV + q] + ix * f.in[Y::ADV + q] * dusx;
+#pragma unroll
+        for (int v = 0; v < S; ++v) r[v] = r[v] + iy * y_part(v, false, iy);
+#pragma unroll
+        for (int q = 0; q < NF; ++q) r[Y::ADV + q] = r[Y::ADV + q] + iy * f.in[Y::ADV + q] * dusy;
+        if (a.rk == kRkNone) {
+#pragma unroll
+            for (int v = 0; v < S; ++v) el(out.rhs.v[v], ro) = r[v];
+        } else {
+            double o[S];
+            rk_combine<S>(a, f, r, o);
+#pragma unroll
+            for (int v = 0; v < S; ++v) el(out.qout.v[v], go) = o[v];
+        }
+        return;
+    }
+    if (a.fold) {
+        // spread RK stage: ... + cdt*(L_x + L_y) + ci*in
+        const double sx = a.cdt * ix, sy = a.cdt * iy;
+#pragma unroll
+        for (int v = 0; v < S; ++v) r[v] = __builtin_fma(sx, dfx[v], y_part(v, true, sy));
+#pragma unroll
+        for (int q = 0; q < NF; ++q)
+            r[Y::ADV + q] = r[Y::ADV + q] + (sx * dusx + sy * dusy) * f.in[Y::ADV + q];
+        if (a.ci != 0.0) {
+#pragma unroll
+            for (int v = 0; v < S; ++v) r[v] = r[v] + a.ci * f.in[v];
+        }
+        if constexpr (sizeof(R) == 4) {
+            // FP32 bulk: volume fractions clipped to [0, 1], as finish_cell
+#pragma unroll
+            for (int q = 0; q < NF; ++q) r[Y::ADV + q] = min(max(r[Y::ADV + q], 0.0), 1.0);
+        }
+#pragma unroll
+        for (int v = 0; v < S; ++v) el(out.qout.v[v], go) = r[v];
+    } else {
+#pragma unroll
+        for (int v = 0; v < S; ++v) r[v] = __builtin_fma(ix, dfx[v], y_part(v, false, iy));
+#pragma unroll
+        for (int q = 0; q < NF; ++q)
+            r[Y::ADV + q] = r[Y::ADV + q] + (ix * dusx + iy * dusy) * f.in[Y::ADV + q];
+#pragma unroll
+        for (int v = 0; v < S; ++v) el(out.rhs.v[v], ro) = r[v];
     }
 }
 
@@ -1370,74 +1467,20 @@ __global__ __launch_bounds__(kXyThreads) __attribute__((amdgpu_waves_per_eu(4, 8
         }
         const double dusy = to_d(fyl[S][xr + 1][yc]) - to_d(fyl[S][xr][yc]), dusx = to_d(usx) - to_d(usxm);
         const double ix = a.inv_ds[i], iy = a.inv_ds2[j];
-        double r[S];
+        FinishIn<S> f;
+#pragma unroll
+        for (int v = 0; v < S; ++v) f.in[v] = cin[v];
         if constexpr (!kFastF64 && sizeof(R) == 8) {
-            // plain FP64: the x sweep's finish (the first direction: it
-            // assigns) and then the y sweep's, operation for operation, so
-            // the result is bitwise theirs; then the rhs store or the RK
-            // stage (2D, where y is the last direction)
+            if (a.rk != kRkNone) {
 #pragma unroll
-            for (int v = 0; v < S; ++v) r[v] = ix * dfx[v];
-#pragma unroll
-            for (int q = 0; q < NF; ++q) r[Y::ADV + q] = r[Y::ADV + q] + ix * cin[Y::ADV + q] * dusx;
-#pragma unroll
-            for (int v = 0; v < S; ++v) r[v] = r[v] + iy * dfy[v];
-#pragma unroll
-            for (int q = 0; q < NF; ++q) r[Y::ADV + q] = r[Y::ADV + q] + iy * cin[Y::ADV + q] * dusy;
-            if (a.rk == kRkNone) {
-#pragma unroll
-                for (int v = 0; v < S; ++v) el(a.rhs.v[v], ro) = r[v];
-            } else {
-                FinishIn<S> f;
-#pragma unroll
-                for (int v = 0; v < S; ++v) {
-                    f.in[v] = cin[v];
-                    f.base[v] = a.base_is_in ? cin[v] : el(a.qbase.v[v], go);
-                }
-                double o[S];
-                rk_combine<S>(a, f, r, o);
-#pragma unroll
-                for (int v = 0; v < S; ++v) el(a.qout.v[v], go) = o[v];
+                for (int v = 0; v < S; ++v) f.base[v] = a.base_is_in ? cin[v] : el(a.qbase.v[v], go);
             }
-            return;
         }
-        if (a.fold) {
-            // spread RK stage: rhs (z's part in 3D) + the rest of cb*base +
-            // cdt*(L_x + L_y) + ci*in
-            const double sx = a.cdt * ix, sy = a.cdt * iy;
-#pragma unroll
-            for (int v = 0; v < S; ++v) {
-                double acc = a.accumulate ? el(a.rhs.v[v], ro) : 0.0;
-                if (v >= a.base_lo && v < a.base_hi) acc = fma(a.cb, el(a.qbase.v[v], go), acc);
-                acc = fma(sy, dfy[v], acc);
-                r[v] = fma(sx, dfx[v], acc);
-            }
-#pragma unroll
-            for (int q = 0; q < NF; ++q)
-                r[Y::ADV + q] = r[Y::ADV + q] + (sx * dusx + sy * dusy) * cin[Y::ADV + q];
-            if (a.ci != 0.0) {
-#pragma unroll
-                for (int v = 0; v < S; ++v) r[v] = r[v] + a.ci * cin[v];
-            }
-            if constexpr (sizeof(R) == 4) {
-                // FP32 bulk: volume fractions clipped to [0, 1], as finish_cell
-#pragma unroll
-                for (int q = 0; q < NF; ++q) r[Y::ADV + q] = min(max(r[Y::ADV + q], 0.0), 1.0);
-            }
-#pragma unroll
-            for (int v = 0; v < S; ++v) el(a.qout.v[v], go) = r[v];
-        } else {
-#pragma unroll
-            for (int v = 0; v < S; ++v) {
-                const double acc = a.accumulate ? el(a.rhs.v[v], ro) : 0.0;
-                r[v] = acc + iy * dfy[v] + ix * dfx[v];
-            }
-#pragma unroll
-            for (int q = 0; q < NF; ++q)
-                r[Y::ADV + q] = r[Y::ADV + q] + (ix * dusx + iy * dusy) * cin[Y::ADV + q];
-#pragma unroll
-            for (int v = 0; v < S; ++v) el(a.rhs.v[v], ro) = r[v];
-        }
+        finish_xy<NF, D, R>(a, a, go, ro, ix, iy, dfx, dusx, dusy, f, [&](int v, bool fold, double sy) {
+            return finish_y_part<R>(
+                a, fold, sy, dfy[v], v >= a.base_lo && v < a.base_hi, [&] { return el(a.rhs.v[v], ro); },
+                [&] { return el(a.qbase.v[v], go); });
+        });
     }
 }
 
