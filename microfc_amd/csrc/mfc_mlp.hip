@@ -8,6 +8,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -21,6 +22,7 @@ namespace {
 
 constexpr int kTrainBlocksMax = 512;
 constexpr int kRed = kMlpParams + 1; // gradient entries + the loss
+constexpr int kSumP = 64, kSumG = 16; // k_mlp_update: parameters per block, threads per parameter
 
 thread_local std::string g_mlp_err;
 
@@ -45,6 +47,10 @@ struct MlpState {
     float *params = nullptr, *m1 = nullptr, *m2 = nullptr;
     float *partials = nullptr, *grad = nullptr;
     MlpFrags *frags = nullptr;
+    // pinned, kRed floats: what goes to the host (parameters or gradient; the
+    // loss last), one call at a time
+    float *host = nullptr;
+    std::mutex host_use;
     long step = 0;
     hipStream_t stream = nullptr;
 } M;
@@ -278,26 +284,78 @@ __global__ __launch_bounds__(256) void k_mlp_train(const float *S, long n, const
         partials[(long)blockIdx.x * kRed + p] = red[0][p] + red[1][p] + red[2][p] + red[3][p];
 }
 
-// Sums block partials in block order: grad[p] = sum_b partials[b][p];
-// grad[kMlpParams] is the loss (mean of squared errors).
-__global__ void k_mlp_reduce(const float *partials, int nblk, long n, float *grad) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= kRed) return;
-    float s = 0.f;
-    for (int b = 0; b < nblk; ++b) s += partials[(long)b * kRed + p];
-    grad[p] = p == kMlpParams ? s / (float)n : s;
+// Where parameter p (value v) is kept in the packed operands: the inverse of
+// k_mlp_pack's layout, parameter by parameter.
+__device__ __forceinline__ void mlp_scatter(MlpFrags *F, int p, float v) {
+    const short h = (short)f2bf(v);
+    // entry (k, j) of a 16 x 16 operand tile is element k%4 of lane j + 16*(k/4)
+    auto at = [](int k, int j) { return j + 16 * (k >> 2); };
+    if (p < kOffB1) {
+        const int r = p >> 5, c = p & 31;
+        F->w1[c >> 4][at(r, c & 15)][r & 3] = h;
+    } else if (p < kOffW2) {
+        const int i = p - kOffB1;
+        F->b1[i] = v;
+        for (int j = 0; j < 16; ++j) F->c1[i >> 4][at(i & 15, j)][i & 3] = v;
+    } else if (p < kOffB2) {
+        const int r = (p - kOffW2) >> 5, c = (p - kOffW2) & 31;
+        F->w2[r >> 4][c >> 4][at(r & 15, c & 15)][r & 3] = h;
+        F->w2t[c >> 4][r >> 4][at(c & 15, r & 15)][c & 3] = h;
+    } else if (p < kOffW3) {
+        const int i = p - kOffB2;
+        F->b2[i] = v;
+        for (int j = 0; j < 16; ++j) F->c2[i >> 4][at(i & 15, j)][i & 3] = v;
+    } else if (p < kOffB3) {
+        const int r = (p - kOffW3) >> 4, c = (p - kOffW3) & 15;
+        F->w3[r >> 4][at(r & 15, c)][r & 3] = h;
+        F->w3t[r >> 4][at(c, r & 15)][c & 3] = h;
+        if (c < kMlpOut)
+            for (int q = 0; q < 4; ++q) F->w3q[q][r >> 4][at(r & 15, c + 4 * q)][r & 3] = h;
+    } else {
+        F->b3[p - kOffB3] = v;
+    }
 }
 
-__global__ void k_mlp_adam(const float *grad, float *P, float *m1, float *m2, float lr, float b1, float b2,
-                           float eps, float c1, float c2) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= kMlpParams) return;
-    const float g = grad[p];
-    const float a = b1 * m1[p] + (1.f - b1) * g;
-    const float v = b2 * m2[p] + (1.f - b2) * g * g;
-    m1[p] = a;
-    m2[p] = v;
-    P[p] -= lr * (a / c1) / (sqrtf(v / c2) + eps);
+// Sums the block partials, grad[p] = sum_b partials[b][p] (p = kMlpParams:
+// the loss, a mean), and with ADAM updates the parameter, its moments and its
+// packed operands; the loss also goes to pinned host memory.  A block takes
+// kSumP parameters, kSumG threads each, with every thread's partials
+// kSumG blocks apart and eight loads in flight.  (4.4 MB at 512 partials: one
+// thread per parameter walking them one after another took 115 us, and the
+// Adam step and the packing a launch each, 2.4 and 6.9 us.)
+template <bool ADAM>
+__global__ __launch_bounds__(kSumP *kSumG) void k_mlp_update(const float *partials, int nblk, long n, float *grad,
+                                                             float *host_loss, float *P, float *m1, float *m2,
+                                                             MlpFrags *F, float lr, float b1, float b2, float eps,
+                                                             float c1, float c2) {
+    __shared__ float red[kSumG][kSumP];
+    const int lane = threadIdx.x % kSumP, g = threadIdx.x / kSumP;
+    const int p = blockIdx.x * kSumP + lane;
+    float s = 0.f;
+    if (p < kRed) {
+#pragma unroll 8
+        for (int b = g; b < nblk; b += kSumG) s += partials[(long)b * kRed + p];
+    }
+    red[g][lane] = s;
+    __syncthreads();
+    if (g != 0 || p >= kRed) return;
+#pragma unroll
+    for (int k = 1; k < kSumG; ++k) s += red[k][lane];
+    if (p == kMlpParams) {
+        grad[p] = s / (float)n;
+        *host_loss = s / (float)n;
+        return;
+    }
+    grad[p] = s;
+    if constexpr (ADAM) {
+        const float a = b1 * m1[p] + (1.f - b1) * s;
+        const float v = b2 * m2[p] + (1.f - b2) * s * s;
+        m1[p] = a;
+        m2[p] = v;
+        const float w = P[p] - lr * (a / c1) / (sqrtf(v / c2) + eps);
+        P[p] = w;
+        mlp_scatter(F, p, w);
+    }
 }
 
 // Inference: out has 4 planes of n floats (w0, w1, w2, learned face value in
@@ -479,18 +537,27 @@ int mlp_pack() {
     return 0;
 }
 
-int mlp_grad(const float *samples, long n, float *loss) {
+// The gradient of n samples into M.grad, and the loss into M.host; with lr > 0
+// also one Adam step.
+int mlp_grad(const float *samples, long n, float lr) {
     if (n <= 0) return mfail(-1, "no samples");
     const long ntile = (n + 15) / 16;
     const int nblk = (int)std::min<long>(kTrainBlocksMax, (ntile + 3) / 4);
     hipLaunchKernelGGL(k_mlp_train, dim3(nblk), dim3(256), 0, M.stream, samples, n, M.frags, M.partials);
     MHIP(hipGetLastError());
-    hipLaunchKernelGGL(k_mlp_reduce, dim3((kRed + 255) / 256), dim3(256), 0, M.stream, M.partials, nblk, n, M.grad);
-    MHIP(hipGetLastError());
-    if (loss) {
-        MHIP(hipMemcpyAsync(loss, M.grad + kMlpParams, sizeof(float), hipMemcpyDeviceToHost, M.stream));
-        MHIP(hipStreamSynchronize(M.stream));
+    const dim3 grid((kRed + kSumP - 1) / kSumP), block(kSumP * kSumG);
+    float *loss = M.host + kMlpParams;
+    if (lr > 0.f) {
+        const float b1 = 0.9f, b2 = 0.999f, t = (float)(M.step + 1);
+        const float c1 = 1.f - powf(b1, t), c2 = 1.f - powf(b2, t);
+        hipLaunchKernelGGL(k_mlp_update<true>, grid, block, 0, M.stream, M.partials, nblk, n, M.grad, loss, M.params,
+                           M.m1, M.m2, M.frags, lr, b1, b2, 1e-8f, c1, c2);
+    } else {
+        hipLaunchKernelGGL(k_mlp_update<false>, grid, block, 0, M.stream, M.partials, nblk, n, M.grad, loss, M.params,
+                           M.m1, M.m2, M.frags, lr, 0.f, 0.f, 0.f, 1.f, 1.f);
     }
+    MHIP(hipGetLastError());
+    if (lr > 0.f) M.step += 1;
     return 0;
 }
 
@@ -515,6 +582,7 @@ int mfc_mlp_init(const float *params) {
         MHIP(hipMalloc(&M.grad, sizeof(float) * kRed));
         MHIP(hipMalloc(&M.partials, sizeof(float) * kRed * kTrainBlocksMax));
         MHIP(hipMalloc(&M.frags, sizeof(MlpFrags)));
+        MHIP(hipHostMalloc(&M.host, sizeof(float) * kRed, hipHostMallocDefault));
         M.init = true;
     }
     MHIP(hipMemcpyAsync(M.params, params, sizeof(float) * kMlpParams, hipMemcpyHostToDevice, M.stream));
@@ -528,33 +596,32 @@ int mfc_mlp_init(const float *params) {
 
 int mfc_mlp_get(float *params) {
     if (int rc = mlp_require()) return rc;
-    MHIP(hipMemcpyAsync(params, M.params, sizeof(float) * kMlpParams, hipMemcpyDeviceToHost, M.stream));
+    std::lock_guard<std::mutex> use(M.host_use);
+    MHIP(hipMemcpyAsync(M.host, M.params, sizeof(float) * kMlpParams, hipMemcpyDeviceToHost, M.stream));
     MHIP(hipStreamSynchronize(M.stream));
+    memcpy(params, M.host, sizeof(float) * kMlpParams);
     return 0;
 }
 
 int mfc_mlp_gradient(const float *samples, long n, float *grad, float *loss) {
     if (int rc = mlp_require()) return rc;
-    if (int rc = mlp_grad(samples, n, loss)) return rc;
-    if (grad) {
-        MHIP(hipMemcpyAsync(grad, M.grad, sizeof(float) * kMlpParams, hipMemcpyDeviceToHost, M.stream));
-        MHIP(hipStreamSynchronize(M.stream));
-    }
+    std::lock_guard<std::mutex> use(M.host_use);
+    if (int rc = mlp_grad(samples, n, 0.f)) return rc;
+    if (grad)
+        MHIP(hipMemcpyAsync(M.host, M.grad, sizeof(float) * kMlpParams, hipMemcpyDeviceToHost, M.stream));
+    if (grad || loss) MHIP(hipStreamSynchronize(M.stream));
+    if (grad) memcpy(grad, M.host, sizeof(float) * kMlpParams);
+    if (loss) *loss = M.host[kMlpParams];
     return 0;
 }
 
 int mfc_mlp_train_step(const float *samples, long n, float lr, float *loss) {
     if (int rc = mlp_require()) return rc;
     if (!(lr > 0.f)) return mfail(-1, "learning rate must be positive");
-    if (int rc = mlp_grad(samples, n, loss)) return rc;
-    M.step += 1;
-    const float b1 = 0.9f, b2 = 0.999f;
-    const float c1 = 1.f - powf(b1, (float)M.step), c2 = 1.f - powf(b2, (float)M.step);
-    hipLaunchKernelGGL(k_mlp_adam, dim3((kMlpParams + 255) / 256), dim3(256), 0, M.stream, M.grad, M.params, M.m1,
-                       M.m2, lr, b1, b2, 1e-8f, c1, c2);
-    MHIP(hipGetLastError());
-    if (int rc = mlp_pack()) return rc;
+    std::lock_guard<std::mutex> use(M.host_use);
+    if (int rc = mlp_grad(samples, n, lr)) return rc;
     MHIP(hipStreamSynchronize(M.stream));
+    if (loss) *loss = M.host[kMlpParams];
     return 0;
 }
 
