@@ -368,50 +368,55 @@ __device__ __forceinline__ int bc_source(int bcb, int bce, int s, int i, bool &f
 // fills one ghost cell with that composed map.  blockIdx.y selects the slab:
 // 0: x ghosts (all j, k), 1: y ghosts (interior i, all k), 2: z ghosts
 // (interior i, j); together they cover every ghost cell once.
-__global__ void k_bc_fill(Fields q, int S, int momxb, Box x, int bxb, int bxe, int byb, int bye, int bzb,
-                          int bze, long n0, long n1, long n2) {
+//
+// Latency bound on small grids (a few thousand ghost cells): every variable's
+// load is issued before the first store (one variable after another, each
+// round trip waits for the one before), and the cell's indices come from
+// 32-bit divisions.  200 x 150 cells, 7 variables 4.7 -> 3.7 us, 1000 cells 3.3 -> 2.8 us.
+constexpr int kBcVars = 8; // variables per round trip
+__global__ __launch_bounds__(256) void k_bc_fill(Fields q, int S, int momxb, Box x, int bxb, int bxe, int byb, int bye,
+                                                 int bzb, int bze, unsigned n0, unsigned n1, unsigned n2) {
     const int slab = blockIdx.y;
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const unsigned t = blockIdx.x * 256u + threadIdx.x;
     int i, j, k;
-    const int gx = 2 * x.b, gy = 2 * x.bj;
-    const int NY = x.n + 1 + gy, NX = x.m + 1;
+    const unsigned gx = 2 * x.b, gy = 2 * x.bj;
+    const unsigned NY = x.n + 1 + gy, NX = x.m + 1;
     if (slab == 0) {
         if (t >= n0) return;
-        const int gi = (int)(t % gx);
-        const long r = t / gx;
-        const int jj = (int)(r % NY);
-        const int kk = (int)(r / NY);
-        i = gi < x.b ? gi - x.b : x.m + 1 + (gi - x.b);
-        j = jj - x.bj;
-        k = kk - x.bk;
+        const unsigned r = t / gx, gi = t - r * gx, kk = r / NY, jj = r - kk * NY;
+        i = (int)gi < x.b ? (int)gi - x.b : x.m + 1 + ((int)gi - x.b);
+        j = (int)jj - x.bj;
+        k = (int)kk - x.bk;
     } else if (slab == 1) {
         if (t >= n1) return;
-        const int ii = (int)(t % NX);
-        const long r = t / NX;
-        const int gj = (int)(r % gy);
-        const int kk = (int)(r / gy);
-        i = ii;
-        j = gj < x.bj ? gj - x.bj : x.n + 1 + (gj - x.bj);
-        k = kk - x.bk;
+        const unsigned r = t / NX, ii = t - r * NX, kk = r / gy, gj = r - kk * gy;
+        i = (int)ii;
+        j = (int)gj < x.bj ? (int)gj - x.bj : x.n + 1 + ((int)gj - x.bj);
+        k = (int)kk - x.bk;
     } else {
         if (t >= n2) return;
-        const int ii = (int)(t % NX);
-        const long r = t / NX;
-        const int jj = (int)(r % (x.n + 1));
-        const int gk = (int)(r / (x.n + 1));
-        i = ii;
-        j = jj;
-        k = gk < x.bk ? gk - x.bk : x.p + 1 + (gk - x.bk);
+        const unsigned r = t / NX, ii = t - r * NX, NI = x.n + 1, gk = r / NI, jj = r - gk * NI;
+        i = (int)ii;
+        j = (int)jj;
+        k = (int)gk < x.bk ? (int)gk - x.bk : x.p + 1 + ((int)gk - x.bk);
     }
     bool fx = false, fy = false, fz = false;
     const int si = bc_source(bxb, bxe, x.m, i, fx);
     const int sj = x.bj ? bc_source(byb, bye, x.n, j, fy) : j;
     const int sk = x.bk ? bc_source(bzb, bze, x.p, k, fz) : k;
     const long dst = box_off(x, i, j, k), src = box_off(x, si, sj, sk);
-    for (int v = 0; v < S; ++v) {
-        double val = q.v[v][src];
-        if ((fx && v == momxb) || (fy && v == momxb + 1) || (fz && v == momxb + 2)) val = -val;
-        q.v[v][dst] = val;
+    for (int v0 = 0; v0 < S; v0 += kBcVars) {
+        double val[kBcVars];
+#pragma unroll
+        for (int u = 0; u < kBcVars; ++u)
+            if (v0 + u < S) val[u] = q.v[v0 + u][src];
+#pragma unroll
+        for (int u = 0; u < kBcVars; ++u) {
+            const int v = v0 + u;
+            if (v >= S) break;
+            const bool neg = (fx && v == momxb) || (fy && v == momxb + 1) || (fz && v == momxb + 2);
+            q.v[v][dst] = neg ? -val[u] : val[u];
+        }
     }
 }
 
@@ -690,7 +695,8 @@ int bc_fill(const Fields &q) {
     const dim3 grid((unsigned)((nmax + 255) / 256), 1 + (G.D >= 2) + (G.D >= 3)), block(256);
     TimedScope ts(kKBcFill);
     hipLaunchKernelGGL(k_bc_fill, grid, block, 0, G.stream, q, G.S, G.prm.num_fluids, x, G.prm.bc_x_beg,
-                       G.prm.bc_x_end, G.prm.bc_y_beg, G.prm.bc_y_end, G.prm.bc_z_beg, G.prm.bc_z_end, n0, n1, n2);
+                       G.prm.bc_x_end, G.prm.bc_y_beg, G.prm.bc_y_end, G.prm.bc_z_beg, G.prm.bc_z_end, (unsigned)n0,
+                       (unsigned)n1, (unsigned)n2);
     HIPCHK(hipGetLastError());
     return 0;
 }
