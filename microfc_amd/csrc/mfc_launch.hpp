@@ -33,7 +33,14 @@ int launch_sweep(const SweepLaunch &L, const SweepArgs &a, hipStream_t st);
             if constexpr (NF <= kMarchMaxFluids && D == 3 && WO == 5 && !ML) hipLaunchKernelGGL((k_march<NF, 3, 2, R, false, UNI>), grid, dim3(64), 0, st, a); \
             else return -1;                                                                             \
         } else if (dir == 3) {                                                                          \
-            if constexpr (NF <= kXyMaxFluids && D >= 2 && WO == 5 && !ML && UNI) hipLaunchKernelGGL((k_sweep_xy<NF, D, R>), grid, dim3(kXyThreads), 0, st, a); \
+            if constexpr (NF <= kXyMaxFluids && D >= 2 && WO == 5 && !ML && UNI) {                      \
+                if constexpr (D == 2 && sizeof(R) == 8)                                                 \
+                    if (a.ghosts) {                                                                     \
+                        hipLaunchKernelGGL((k_sweep_xy<NF, D, R, true>), grid, dim3(kXyThreads), 0, st, a); \
+                        return hipGetLastError() == hipSuccess ? 0 : -2;                                \
+                    }                                                                                   \
+                hipLaunchKernelGGL((k_sweep_xy<NF, D, R, false>), grid, dim3(kXyThreads), 0, st, a);    \
+            }                                                                                           \
             else return -1;                                                                             \
         } else if (dir == 0) {                                                                          \
             hipLaunchKernelGGL((k_sweep_x<NF, D, WO, R, ML, UNI>), grid, dim3(64), 0, st, a);                \

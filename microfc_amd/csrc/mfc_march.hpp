@@ -343,7 +343,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(march_waves<
                         march_prim_in<NF, D, R, FM>(args(), pv, fin);
                     }
                     if (finish)
-                        finish_cell<NF, D, R, FM>(args(), go, ro, a.inv_ds[jr], fl, f, usl, us, fin, BLO, BHI);
+                        finish_cell<NF, D, R, FM, false>(args(), go, ro, a.inv_ds[jr], fl, f, usl, us, fin, BLO, BHI, x, t, jr);
                 } else {
                     // 2. x faces of row jr
                     const double iy = a.inv_ds2[jr];
@@ -408,7 +408,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(march_waves<
                     for (int v = 0; v < NK; ++v) fin.in[Y::MOM + v] = ko[v];
                     if (finish) march_prim_in<NF, D, R, FM>(args(), w0, fin);
                     if (finish)
-                        finish_xy<NF, D, R>(args(), fresh_args(), go, ro, ix, iy, dfx, dux, duy, fin,
+                        finish_xy<NF, D, R, false>(args(), fresh_args(), go, ro, ix, iy, dfx, dux, duy, fin, x, jr, t,
                                             [&](int v, bool, double) { return acc[v]; });
                 }
             }

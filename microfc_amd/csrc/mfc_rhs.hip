@@ -732,6 +732,7 @@ SweepArgs sweep_args(int d) {
                            {G.prm.bc_z_beg, G.prm.bc_z_end}};
     a.bc_beg = bcs[d][0];
     a.bc_end = bcs[d][1];
+    memcpy(a.bcs, bcs, sizeof bcs);
     a.uniform = G.dir[d].uniform ? 1 : 0;
     for (int q = 0; q < kNCoef; ++q) {
         a.ucf[q] = G.dir[d].ucf[q];
@@ -907,11 +908,22 @@ int viscous(int d, const Fields &qin, const Fields &rhs, const SweepArgs &sa) {
     return 0;
 }
 
+// Whether the sweep that writes an RK stage fills the stage's ghost cells.
+bool sweeps_fill_ghosts() {
+    if (G.visc || G.D > 2) return false;
+    if (G.D == 1 || G.prm.precision == MFC_PREC_FP32_LEARNED) return true;
+    return G.prm.precision != MFC_PREC_FP32_BULK && kFuseXY && G.prm.weno_order == 5 &&
+           G.prm.num_fluids <= kXyMaxFluids && G.dir[0].uniform && G.dir[1].uniform && !marches(4);
+}
+
 // All directional sweeps of one RHS evaluation on the ghost-filled field qin.
 // The last sweep either writes rhs (rk = kRkNone) or applies the RK stage.
 // Viscous runs use the viscous kernels for each direction instead, with the
 // same finish semantics.
-int sweeps(const Fields &qin, const Fields &rhs, int rk, const Fields *qbase, const Fields *qout, double dt) {
+// ghosts: the last sweep also fills the ghost cells of *qout (the caller's
+// next stage input; sweeps_fill_ghosts).
+int sweeps(const Fields &qin, const Fields &rhs, int rk, const Fields *qbase, const Fields *qout, double dt,
+           bool ghosts = false) {
     // The plain form adds the directions in the reference's order x, y, z
     // (m_rhs.fpp:469-656; it fixes the rounding).  The contracted FP64,
     // FP32-bulk and learned forms run them in the reverse order: the sum is
@@ -983,6 +995,7 @@ int sweeps(const Fields &qin, const Fields &rhs, int rk, const Fields *qbase, co
             a.rhs = rhs;
             a.dt = dt;
             a.rk = kRkNone;
+            a.ghosts = ghosts && fold_kind == 3;
             if (fold) {
                 a.qbase = *qbase;
                 a.qout = *qout;
@@ -1017,6 +1030,7 @@ int sweeps(const Fields &qin, const Fields &rhs, int rk, const Fields *qbase, co
             a.rhs = rhs;
             a.dt = dt;
             a.rk = last ? rk : kRkNone;
+            a.ghosts = ghosts && last;
             if (a.rk != kRkNone) {
                 a.qbase = *qbase;
                 a.qout = *qout;
@@ -1044,6 +1058,7 @@ int sweeps(const Fields &qin, const Fields &rhs, int rk, const Fields *qbase, co
         a.dt = dt;
         const bool last = k == G.D - 1;
         a.rk = last && !fold ? rk : kRkNone;
+        a.ghosts = ghosts && last;
         if (a.rk != kRkNone || fold) {
             a.qbase = *qbase;
             a.qout = *qout;
@@ -1251,9 +1266,14 @@ int mfc_tvd_rk_step(int t_step, double dt, double *const *q_cons_ts1, double *co
         HIPCHK(hipGetLastError());
         return 0;
     }
+    // a stage whose output is the next stage's input, with its ghost cells
+    const bool filled = sweeps_fill_ghosts();
+    auto stage = [&](const Fields &in, int rk, const Fields &out) -> int {
+        if (int rc = sweeps(in, rhs, rk, &q1, &out, dt, filled)) return rc;
+        return filled ? 0 : bc_fill(out);
+    };
     if (G.prm.time_stepper == 2) {
-        if (int rc = sweeps(q1, rhs, kRkEuler, &q1, &q2, dt)) return rc;
-        if (int rc = bc_fill(q2)) return rc;
+        if (int rc = stage(q1, kRkEuler, q2)) return rc;
         return sweeps(q2, rhs, kRk2Final, &q1, &q1, dt);
     }
     if (!G.scratch_state) HIPCHK(hipMalloc(&G.scratch_state, sizeof(double) * G.S * G.ng));
@@ -1262,10 +1282,8 @@ int mfc_tvd_rk_step(int t_step, double dt, double *const *q_cons_ts1, double *co
     // stage 1: q3 = q1 + dt*L(q1); stage 2: q2 = (3 q1 + q3 + dt*L(q3))/4;
     // stage 3: q1 = (q1 + 2 q2 + 2 dt*L(q2))/3.  Each stage reads its input's
     // stencil and writes a different array, or only its own cell of q1.
-    if (int rc = sweeps(q1, rhs, kRkEuler, &q1, &q3, dt)) return rc;
-    if (int rc = bc_fill(q3)) return rc;
-    if (int rc = sweeps(q3, rhs, kRk3Stage2, &q1, &q2, dt)) return rc;
-    if (int rc = bc_fill(q2)) return rc;
+    if (int rc = stage(q1, kRkEuler, q3)) return rc;
+    if (int rc = stage(q3, kRk3Stage2, q2)) return rc;
     return sweeps(q2, rhs, kRk3Stage3, &q1, &q1, dt);
 }
 

@@ -90,6 +90,11 @@ struct SweepArgs {
     const double *coef2;
     long ncell2;
     int rl; // entries per row of the outer index (k_march)
+    // the RK stage's ghost cells: filled with its output by the sweep that
+    // writes it (the stage output is then the next stage's input), from the
+    // boundary codes of every direction
+    int ghosts;
+    int bcs[3][2];
 };
 
 // RK-base variables the z sweep adds before the fused x and y sweep
@@ -280,6 +285,77 @@ __device__ __forceinline__ void finish_load_adv(const SweepArgs &a, Off go, Off 
         if (v >= a.base_lo && v < a.base_hi) f.base[v] = el(a.qbase.v[v], go);
 }
 
+// Ghost cells that copy interior cell i of a direction with last index s,
+// boundary codes bc and b ghost layers: n0 cells from g0 on (mirrored ones
+// with flip0), and n1 from g1 on.
+struct GhostSet {
+    int g0, n0, g1, n1;
+    bool flip0, flip1;
+};
+__device__ __forceinline__ GhostSet ghosts_of(int i, int s, const int *bc, int b) {
+    GhostSet e{0, 0, 0, 0, bc[0] == -2, bc[1] == -2};
+    if (bc[0] <= -3) {
+        if (i == 0) e.g0 = -b, e.n0 = b;
+    } else if (bc[0] == -2) {
+        if (i < b) e.g0 = -i - 1, e.n0 = 1;
+    } else if (i >= s + 1 - b) {
+        e.g0 = i - (s + 1), e.n0 = 1;
+    }
+    if (bc[1] <= -3) {
+        if (i == s) e.g1 = s + 1, e.n1 = b;
+    } else if (bc[1] == -2) {
+        if (i > s - b) e.g1 = 2 * s + 1 - i, e.n1 = 1;
+    } else if (i < b) {
+        e.g1 = i + s + 1, e.n1 = 1;
+    }
+    return e;
+}
+
+// Fills the ghost cells of the stage output that copy cell (i, j, k), whose
+// values are r: every combination of the cell's copies in each direction (the
+// reference's x, then y, then z fill), the momentum normal to a mirror
+// negated.  Saves a pass of k_bc_fill and its launch per RK stage after the
+// first (RK3 step of 1000 cells: 30.0 -> 27.9 us; 768 x 768, contracted 188 ->
+// 176 us; 1024 x 1024 learned 514 -> 507 us).
+template <int NF, int D>
+__device__ __forceinline__ void store_ghosts(const SweepArgs &a, const SweepArgs &out, int i, int j, int k,
+                                             const double *r) {
+    using Y = Sys<NF, D>;
+    constexpr int S = Y::S;
+    if (!a.ghosts) return;
+    bool edge = i < a.b || i > a.m - a.b;
+    if constexpr (D > 1) edge = edge || j < a.b || j > a.n - a.b;
+    if constexpr (D > 2) edge = edge || k < a.b || k > a.p - a.b;
+    if (!edge) return;
+    const GhostSet none{0, 0, 0, 0, false, false};
+    const GhostSet ex = ghosts_of(i, a.m, a.bcs[0], a.b);
+    const GhostSet ey = D > 1 ? ghosts_of(j, a.n, a.bcs[1], a.b) : none;
+    const GhostSet ez = D > 2 ? ghosts_of(k, a.p, a.bcs[2], a.b) : none;
+    // copy c of a direction: the cell itself, then the lower, then the upper
+    // ghosts
+    auto copy = [](const GhostSet &e, int c, int own, bool &flip) {
+        flip = c == 0 ? false : c <= e.n0 ? e.flip0 : e.flip1;
+        return c == 0 ? own : c <= e.n0 ? e.g0 + c - 1 : e.g1 + c - 1 - e.n0;
+    };
+#pragma unroll 1
+    for (int ck = 0; ck <= ez.n0 + ez.n1; ++ck) {
+#pragma unroll 1
+        for (int cj = 0; cj <= ey.n0 + ey.n1; ++cj) {
+#pragma unroll 1
+            for (int ci = cj == 0 && ck == 0 ? 1 : 0; ci <= ex.n0 + ex.n1; ++ci) {
+                bool f[3];
+                const int gi = copy(ex, ci, i, f[0]), gj = copy(ey, cj, j, f[1]), gk = copy(ez, ck, k, f[2]);
+                const long o = ghost_off(a, gi, gj, gk);
+#pragma unroll
+                for (int v = 0; v < S; ++v) {
+                    const bool neg = v >= Y::MOM && v < Y::MOM + D && f[v - Y::MOM];
+                    out.qout.v[v][o] = neg ? -r[v] : r[v];
+                }
+            }
+        }
+    }
+}
+
 // x/3 of the third RK3 stage: the IEEE quotient in the plain form, a
 // multiply by the rounded 1/3 in the contracted FP64 form.
 __device__ __forceinline__ double third(double x) {
@@ -315,10 +391,10 @@ __device__ __forceinline__ void rk_combine(const SweepArgs &a, const FinishIn<S>
 
 // Finishes one cell: flux divergence, alpha*div(u) source, then either the
 // rhs store or the fused RK stage (m_rhs.fpp:565-652, m_time_steppers.fpp).
-template <int NF, int D, typename R, int M, typename O>
+template <int NF, int D, typename R, int M, bool GH, typename O>
 __device__ __forceinline__ void finish_cell(const SweepArgs &a, O go, O ro, double inv,
                                             const R *Fm, const R *Fp, R usm, R usp,
-                                            const FinishIn<Sys<NF, D>::S> &f, int lo, int hi) {
+                                            const FinishIn<Sys<NF, D>::S> &f, int lo, int hi, int i, int j, int k) {
     using Y = Sys<NF, D>;
     constexpr int S = Y::S;
     double r[S];
@@ -361,6 +437,7 @@ __device__ __forceinline__ void finish_cell(const SweepArgs &a, O go, O ro, doub
             }
 #pragma unroll
             for (int v = 0; v < S; ++v) el(a.qout.v[v], go) = r[v];
+            if constexpr (GH) store_ghosts<NF, D>(a, a, i, j, k, r);
             return;
         }
     }
@@ -371,25 +448,32 @@ __device__ __forceinline__ void finish_cell(const SweepArgs &a, O go, O ro, doub
     }
 #pragma unroll
     for (int i = 0; i < NF; ++i) r[Y::ADV + i] = r[Y::ADV + i] + inv * f.in[Y::ADV + i] * dus;
-    if constexpr (!std::is_same<R, double>::value) {
-        // FP32 bulk: the RK stage accumulates in FP64 and clips the volume
-        // fractions to [0, 1] (positivity; the reference has no clip).
-        if (a.rk != kRkNone) {
-            double o[S];
-            rk_combine<S>(a, f, r, o);
-#pragma unroll
-            for (int i = 0; i < NF; ++i) o[Y::ADV + i] = min(max(o[Y::ADV + i], 0.0), 1.0);
-#pragma unroll
-            for (int v = 0; v < S; ++v) el(a.qout.v[v], go) = o[v];
-            return;
-        }
-    }
     if constexpr (M != kModesAll) {
         // no RK stage reaches these sweeps
 #pragma unroll
         for (int v = 0; v < S; ++v) el(a.rhs.v[v], ro) = r[v];
         return;
     }
+    const bool stage = a.rk != kRkNone;
+    if constexpr (!std::is_same<R, double>::value || GH) {
+        if (stage) {
+            double o[S];
+            rk_combine<S>(a, f, r, o);
+            // FP32 bulk: the RK stage accumulates in FP64 and clips the
+            // volume fractions to [0, 1] (positivity; the reference has no
+            // clip).
+            if constexpr (!std::is_same<R, double>::value) {
+#pragma unroll
+                for (int q = 0; q < NF; ++q) o[Y::ADV + q] = min(max(o[Y::ADV + q], 0.0), 1.0);
+            }
+#pragma unroll
+            for (int v = 0; v < S; ++v) el(a.qout.v[v], go) = o[v];
+            if constexpr (GH) store_ghosts<NF, D>(a, a, i, j, k, o);
+            return;
+        }
+    }
+    // combined and stored per variable: with the results in an array first,
+    // k_sweep_t kept that array in scratch
     switch (a.rk) {
     case kRkNone:
 #pragma unroll
@@ -570,11 +654,20 @@ constexpr bool x_cell_parallel() { return ML || sizeof(R) == 4 || UNI; }
 template <bool ML, typename R, bool UNI>
 constexpr int x_tile_cells() { return x_cell_parallel<ML, R, UNI>() ? 62 : 63; }
 
+// Whether the x sweep, where it writes an RK stage, fills the stage's ghost
+// cells (store_ghosts): in 1D, and in the learned form's 2D cases.  The
+// values kept past their stores cost registers: in the FP32-bulk x and y sweep
+// (76 -> 90 VGPRs, 1210 x 905 196 -> 215 us per step) and the marches (512^3 x
+// and y 7.4 -> 8.2 ms) more than the ghost fill they save, so those leave it
+// to k_bc_fill, and so does 3D, where a corner cell has 124 copies.
+constexpr bool x_fills_ghosts(int D, bool ml) { return D == 1 || (ml && D == 2); }
+
 template <int NF, int D, int WO, typename R, bool ML, bool UNI>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(ML ? 2 : 4, 8))) void k_sweep_x(const SweepArgs a) {
     using Y = Sys<NF, D>;
     constexpr int S = Y::S;
     constexpr int FM = finish_modes<D, true, R, ML>();
+    constexpr bool GH = x_fills_ghosts(D, ML);
     constexpr int PN = (WO - 1) / 2;
     constexpr int NC = 64 + 2 * PN + 1;
     constexpr int TW = x_tile_cells<ML, R, UNI>();
@@ -752,7 +845,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(ML ? 2 : 4, 
             const Off go{ghost_off(a, x0, j, k), (unsigned)lane}, ro{interior_off(a, x0, j, k), (unsigned)lane};
             FinishIn<S> fin;
             finish_load_staged<NF, D, FM>(a, go, ro, cin, 1, fin);
-            finish_cell<NF, D, R, FM>(a, go, ro, a.inv_ds[i], f, fp, us, usp, fin, a.base_lo, a.base_hi);
+            finish_cell<NF, D, R, FM, GH>(a, go, ro, a.inv_ds[i], f, fp, us, usp, fin, a.base_lo, a.base_hi, i, j, k);
         }
         return;
     }
@@ -788,7 +881,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(ML ? 2 : 4, 
             finish_load_staged<NF, D, FM>(a, go, ro, cin, 1, fin);
         else
             finish_load<NF, D, FM>(a, go, ro, fin);
-        finish_cell<NF, D, R, FM>(a, go, ro, a.inv_ds[i], Fm, Fp, sf[S][lane], sf[S][lane + 1], fin, a.base_lo, a.base_hi);
+        finish_cell<NF, D, R, FM, GH>(a, go, ro, a.inv_ds[i], Fm, Fp, sf[S][lane], sf[S][lane + 1], fin,
+                                  a.base_lo, a.base_hi, i, j, k);
     }
 }
 
@@ -976,8 +1070,8 @@ __global__ __launch_bounds__(t_threads<ML>()) __attribute__((amdgpu_waves_per_eu
             finish_load_staged<NF, D, FM>(a, gcell(i, cc), rcell(i, cc), &lcons[0][ts][tx], (kTS - 1) * kTX, fin);
         else
             finish_load<NF, D, FM>(a, gcell(i, cc), rcell(i, cc), fin);
-        finish_cell<NF, D, R, FM>(a, gcell(i, cc), rcell(i, cc), a.inv_ds[cc], Fm, Fp, sf[S][ts][tx],
-                                  sf[S][ts + 1][tx], fin, a.base_lo, a.base_hi);
+        finish_cell<NF, D, R, FM, false>(a, gcell(i, cc), rcell(i, cc), a.inv_ds[cc], Fm, Fp, sf[S][ts][tx],
+                                  sf[S][ts + 1][tx], fin, a.base_lo, a.base_hi, i, DIR == 1 ? cc : t, DIR == 1 ? t : cc);
     }
 }
 
@@ -1174,7 +1268,8 @@ __global__ __launch_bounds__((tc_cols<R, ML>(DIR) * tc_rows<R>(DIR)))
             finish_load_staged<NF, D, FM>(a, go, ro, &lcons[0][fx][fs], XC * KP, fin);
         else
             finish_load<NF, D, FM>(a, go, ro, fin);
-        finish_cell<NF, D, R, FM>(a, go, ro, a.inv_ds[cc], Fm, Fp, fl[S][fs][fx], fl[S][fs + 1][fx], fin, a.base_lo, a.base_hi);
+        finish_cell<NF, D, R, FM, false>(a, go, ro, a.inv_ds[cc], Fm, Fp, fl[S][fs][fx], fl[S][fs + 1][fx], fin, a.base_lo,
+                                  a.base_hi, i, DIR == 1 ? cc : t, DIR == 1 ? t : cc);
     }
 }
 
@@ -1202,10 +1297,11 @@ __device__ __forceinline__ double finish_y_part(const SweepArgs &a, bool fold, d
 // with the stage input and the plain form's RK base in f: the divergence, the
 // alpha*div(u) sources and the rhs store or the RK stage (out: where the
 // output pointers are read from).
-template <int NF, int D, typename R, typename O, typename YP>
+template <int NF, int D, typename R, bool GH, typename O, typename YP>
 __device__ __forceinline__ void finish_xy(const SweepArgs &a, const SweepArgs &out, O go, O ro, double ix, double iy,
                                           const double *dfx, double dusx, double dusy,
-                                          const FinishIn<Sys<NF, D>::S> &f, YP &&y_part) {
+                                          const FinishIn<Sys<NF, D>::S> &f, int i, int j, int k,
+                                          YP &&y_part) {
     using Y = Sys<NF, D>;
     constexpr int S = Y::S;
     double r[S];
@@ -1230,6 +1326,7 @@ __device__ __forceinline__ void finish_xy(const SweepArgs &a, const SweepArgs &o
             rk_combine<S>(a, f, r, o);
 #pragma unroll
             for (int v = 0; v < S; ++v) el(out.qout.v[v], go) = o[v];
+            if constexpr (GH) store_ghosts<NF, D>(a, out, i, j, k, o);
         }
         return;
     }
@@ -1252,6 +1349,7 @@ __device__ __forceinline__ void finish_xy(const SweepArgs &a, const SweepArgs &o
         }
 #pragma unroll
         for (int v = 0; v < S; ++v) el(out.qout.v[v], go) = r[v];
+        if constexpr (GH) store_ghosts<NF, D>(a, out, i, j, k, r);
     } else {
 #pragma unroll
         for (int v = 0; v < S; ++v) r[v] = __builtin_fma(ix, dfx[v], y_part(v, false, iy));
@@ -1304,7 +1402,9 @@ __device__ __forceinline__ void xy_halo_cell(int h, int &cx, int &ry) {
     }
 }
 
-template <int NF, int D, typename R>
+// GH: fills the stage output's ghost cells (store_ghosts; 2D FP64: 768^2
+// contracted 194 -> 176 us per step with its CFL reduction).
+template <int NF, int D, typename R, bool GH>
 __global__ __launch_bounds__(kXyThreads) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_sweep_xy(const SweepArgs a) {
     static_assert(sizeof(R) == 8 || sizeof(R) == 4, "FP64 or FP32 reconstruction");
     using Y = Sys<NF, D>;
@@ -1476,7 +1576,7 @@ __global__ __launch_bounds__(kXyThreads) __attribute__((amdgpu_waves_per_eu(4, 8
                 for (int v = 0; v < S; ++v) f.base[v] = a.base_is_in ? cin[v] : el(a.qbase.v[v], go);
             }
         }
-        finish_xy<NF, D, R>(a, a, go, ro, ix, iy, dfx, dusx, dusy, f, [&](int v, bool fold, double sy) {
+        finish_xy<NF, D, R, GH>(a, a, go, ro, ix, iy, dfx, dusx, dusy, f, i, j, k, [&](int v, bool fold, double sy) {
             return finish_y_part<R>(
                 a, fold, sy, dfy[v], v >= a.base_lo && v < a.base_hi, [&] { return el(a.rhs.v[v], ro); },
                 [&] { return el(a.qbase.v[v], go); });

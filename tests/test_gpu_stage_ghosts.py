@@ -1,0 +1,71 @@
+"""Ghost cells that the sweeps fill while they write a Runge-Kutta stage (one
+dimension, the learned form in two, and the fused x and y tile in FP64) against
+the FP64 oracle, whose stages are each followed by its own boundary fill: every
+boundary code on every side, in combinations whose corners mix them, on the
+smallest grids of each WENO order and on cell counts that leave partial tiles.
+
+Bars: the plain form is bitwise the oracle's step; the contracted form is
+within 1e-12 (helpers.state_linf); the FP32-bulk and the untrained learned form
+within 1e-3 of each variable's scale, as for their right-hand sides."""
+import numpy as np
+import pytest
+
+from microfc_amd import PREC_FP32_BULK, PREC_FP32_LEARNED, PREC_FP64, PREC_FP64_FAST, RhsModule, ic, learned
+from oracle import oracle as O
+
+from helpers import perturbed, say, state_linf, to_oracle
+
+pytestmark = pytest.mark.gpu
+
+# (beginning, end) codes of x and of y
+BCS = [((-1, -1), (-1, -1)), ((-2, -2), (-2, -2)), ((-3, -4), (-2, -3)), ((-2, -4), (-1, -1)),
+       ((-1, -1), (-4, -2)), ((-4, -2), (-3, -2))]
+GRIDS = [(24, 0, 5, 3), (14, 0, 3, 2), (4, 0, 1, 3), (300, 0, 5, 2), (24, 24, 5, 3), (126, 66, 5, 3), (63, 130, 5, 2)]
+
+
+def _case(m, n, order, stepper, bx, by):
+    prm = ic.shock_bubble_2d(N=32)[0]
+    prm.m, prm.n, prm.weno_order, prm.time_stepper = m, n, order, stepper
+    prm.bc_beg, prm.bc_end = (bx[0], by[0], -3), (bx[1], by[1], -3)
+    g = ic.uniform_grids(prm)
+    X = ic.mesh(prm, g)[0]
+    Y = ic.mesh(prm, g)[1] if n else 0.3 + 0 * X
+    a = 0.5 + 0.4 * np.sin(9 * X + 4 * Y)
+    vel = [30 + 40 * np.sin(7 * Y + X), 25 * np.cos(5 * X) + 20 * Y][:2 if n else 1]
+    prim = np.stack([1000 * a, 1.2 * (1 - a), *vel, 1e6 * (1 + 0.3 * np.cos(11 * X - 3 * Y)), a, 1 - a])
+    return prm, g, perturbed(prm, ic.ghosted(prm, ic.prim_to_cons(prm, prim)), amp=1e-2)
+
+
+@pytest.mark.parametrize("precision", [PREC_FP64, PREC_FP64_FAST, PREC_FP32_BULK, PREC_FP32_LEARNED])
+@pytest.mark.parametrize("m,n,order,stepper", GRIDS)
+def test_step_with_every_boundary(gpu, m, n, order, stepper, precision):
+    if precision == PREC_FP32_LEARNED:
+        if order != 5:
+            pytest.skip("learned weights are for order 5")
+        learned.Mlp()
+    torch = gpu
+    for bx, by in BCS if n else sorted({(b[0], (-3, -3)) for b in BCS}):
+        prm, grids, q = _case(m, n, order, stepper, bx, by)
+        oc = to_oracle(prm)
+        prm.precision = precision
+        mod = RhsModule(prm, grids)
+        try:
+            qd = torch.from_numpy(q.copy()).cuda()
+            q2, rd = mod.new_field(), mod.new_field(ghosted=False)
+            dt = mod.cfl_dt(qd, 0.3)
+            mod.s_tvd_rk(0, (qd, q2), None, rd, dt)
+            mod.sync()
+            got = prm.interior(qd.cpu().numpy())
+            qo = q.copy()
+            O.tvd_rk_step(oc, grids, dt, qo)
+            want = prm.interior(qo)
+            err = state_linf(prm, got, want, q)
+            say(f"[stage ghosts] {m + 1}x{n + 1} order {order} bc {bx} {by} precision {precision} {err.max():.2e}")
+            if precision == PREC_FP64:
+                assert np.array_equal(got, want)
+            elif precision == PREC_FP64_FAST:
+                assert err.max() <= 1e-12
+            else:
+                assert np.all(np.isfinite(got)) and err.max() <= 1e-3
+        finally:
+            mod.finalize()
