@@ -34,7 +34,7 @@ MFC_DECLARE_SWEEPS_WIDE(kFormF64Fast)
 
 using namespace mfc;
 
-constexpr int kReduceBlocks = 8192; // 32 blocks of 256 threads per CU, two cells per thread at 2048^2
+constexpr int kReduceBlocks = 8192; // the stability pass: 32 blocks of 256 threads per CU
 constexpr int kMaxDevices = 64;
 
 // Block partials of the allocation-free CFL reduction (mfc_cfl_dt_noalloc):
@@ -134,6 +134,8 @@ struct State {
     hipStream_t own = nullptr, stream = nullptr;
     double *partials = nullptr; // 2 * kReduceBlocks doubles
     double *scratch = nullptr;  // this device's `scratch` array (kReduceBlocks doubles)
+    unsigned *count = nullptr;  // blocks of the running CFL reduction that are done (k_icfl)
+    double *result = nullptr;   // pinned: its value
     double *scratch_state = nullptr; // S*ng doubles, RK3 stage buffer
     bool visc = false;               // any fluid_pp%Re > 0
     ViscParams vp{};
@@ -478,28 +480,56 @@ __device__ __forceinline__ double icfl_cell(const double *cv, const Eos &eos, co
     }
 }
 
-// Maximum ICFL over the interior and a block max-reduction by wavefront
-// shuffles; block results go to partials[blockIdx.x].  A block takes chunks
-// of 512 consecutive interior cells (x fastest), two per thread with both
-// cells' loads issued before either is converted.
+// Maximum over a block of T threads, valid on its first wave.
+template <int T> __device__ __forceinline__ double block_max(double mx) {
+    __shared__ double red[T / 64];
+    mx = wave_max(mx);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
+    __syncthreads();
+    const double v = wave_max(red[threadIdx.x & (T / 64 - 1)]);
+    __syncthreads(); // red may be written again
+    return v;
+}
+
+// Maximum ICFL over the interior to *result: a block max-reduction by
+// wavefront shuffles into partials[blockIdx.x], and the block that finishes
+// last reduces the partials (count wraps to 0 with it, ready for the next
+// call).  A block takes chunks of kCflChunk consecutive interior cells (x
+// fastest), two per thread with both cells' loads issued before either is
+// converted.  At most two blocks per compute unit: the counter takes 10 ns a
+// block (768^2 cells: 1152 blocks of 256 threads took 37 us with the call).
+// result is pinned host memory.  With the partials reduced by a kernel of
+// their own and the value copied to pageable memory, the call took 34 instead
+// of 24 us (200^2 cells), 38 instead of 30 us (768^2), 210 instead of 197 us
+// (4096^2).
+constexpr int kCflThreads = 512, kCflChunk = 2 * kCflThreads, kCflBlocks = 512;
 template <int NF, int D, bool FROM_CONS>
-__global__ __launch_bounds__(256) void k_icfl(Fields q, Eos eos, Box x, const double *dx, const double *dy,
-                                              const double *dz, double dt, long nint, double *partials) {
+__global__ __launch_bounds__(kCflThreads) void k_icfl(Fields q, Eos eos, Box x, const double *dx, const double *dy,
+                                              const double *dz, double dt, long nint, double *partials,
+                                              unsigned *count, double *result) {
     constexpr int S = Sys<NF, D>::S;
+    const unsigned nx = x.m + 1, ny = x.n + 1;
+    const bool small = nint < (1L << 31); // 32-bit index divisions
     double mx = -INFINITY;
-    for (long c0 = (long)blockIdx.x * 512; c0 < nint; c0 += (long)gridDim.x * 512) {
+    for (long c0 = (long)blockIdx.x * kCflChunk; c0 < nint; c0 += (long)gridDim.x * kCflChunk) {
         double cv[2][S];
         int ci[2], cj[2], ck[2];
         bool ok[2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            const long e = c0 + threadIdx.x + 256 * h;
+            const long e = c0 + threadIdx.x + kCflThreads * h;
             ok[h] = e < nint;
             const long ee = ok[h] ? e : 0;
-            const long r = ee / (x.m + 1);
-            ci[h] = (int)(ee - r * (x.m + 1));
-            cj[h] = (int)(r % (x.n + 1));
-            ck[h] = (int)(r / (x.n + 1));
+            long r;
+            if (small) {
+                r = (unsigned)ee / nx;
+                ck[h] = (int)((unsigned)r / ny);
+            } else {
+                r = ee / nx;
+                ck[h] = (int)(r / ny);
+            }
+            ci[h] = (int)(ee - r * nx);
+            cj[h] = (int)(r - (long)ck[h] * ny);
             const long o = box_off(x, ci[h], cj[h], ck[h]);
 #pragma unroll
             for (int v = 0; v < S; ++v) cv[h][v] = q.v[v][o];
@@ -508,15 +538,23 @@ __global__ __launch_bounds__(256) void k_icfl(Fields q, Eos eos, Box x, const do
         for (int h = 0; h < 2; ++h)
             if (ok[h]) mx = max_nan(mx, icfl_cell<NF, D, FROM_CONS>(cv[h], eos, dx, dy, dz, ci[h], cj[h], ck[h], dt));
     }
-    __shared__ double red[4];
-    mx = wave_max(mx);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
-    __syncthreads();
+    __shared__ bool last;
+    mx = block_max<kCflThreads>(mx);
     if (threadIdx.x == 0) {
-        double v = red[0];
-        for (int w = 1; w < (int)(blockDim.x >> 6); ++w) v = max_nan(v, red[w]);
-        partials[blockIdx.x] = v;
+        // an exchange that has returned is visible to every block: with a
+        // store and a __threadfence (a write-back of L2 per block) instead,
+        // 768^2 cells took 50 us
+        double old = __hip_atomic_exchange(&partials[blockIdx.x], mx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" : "+v"(old) : : "memory");
+        last = atomicInc(count, gridDim.x - 1) == gridDim.x - 1;
     }
+    __syncthreads();
+    if (!last) return;
+    mx = -INFINITY;
+    for (unsigned t = threadIdx.x; t < gridDim.x; t += kCflThreads)
+        mx = max_nan(mx, __hip_atomic_load(&partials[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    mx = block_max<kCflThreads>(mx);
+    if (threadIdx.x == 0) *result = mx;
 }
 
 // Stability criteria of one cell (m_data_output.fpp:214-263) from its
@@ -1120,6 +1158,9 @@ int mfc_rhs_init(const mfc_params *prm) {
     HIPCHK(hipStreamCreateWithFlags(&G.own, hipStreamNonBlocking));
     G.stream = G.own;
     HIPCHK(hipMalloc(&G.partials, sizeof(double) * 2 * kReduceBlocks));
+    HIPCHK(hipMalloc(&G.count, sizeof(unsigned)));
+    HIPCHK(hipMemset(G.count, 0, sizeof(unsigned)));
+    HIPCHK(hipHostMalloc(&G.result, sizeof(double), hipHostMallocDefault));
     {
         int dev = 0;
         HIPCHK(hipGetDevice(&dev));
@@ -1296,7 +1337,7 @@ int mfc_cons_to_prim(double *const *q_cons_vf, double *const *q_prim_vf) {
 }
 
 // The ICFL max-reduction into `partials` (capacity doubles), a grid-stride
-// pass of at most kReduceBlocks blocks, so every grid size fits.  `timed`
+// pass of at most kCflBlocks blocks, so every grid size fits.  `timed`
 // records HIP events around the pass (event creation may allocate, so the
 // allocation-free entry point passes false).
 static int icfl_reduce(double *const *q, bool from_cons, double dt, double *out, double *partials, int capacity,
@@ -1308,28 +1349,23 @@ static int icfl_reduce(double *const *q, bool from_cons, double dt, double *out,
     const Box x = box();
     const Eos e = eos();
     double *dxs[3] = {G.dir[0].ds_dev, G.dir[1].ds_dev, G.dir[2].ds_dev};
-    const int nb = (int)std::min<long>(kReduceBlocks, std::max<long>(1, (G.nint + 511) / 512));
+    const int nb = (int)std::min<long>(kCflBlocks, (G.nint + kCflChunk - 1) / kCflChunk);
     if (!partials || nb > capacity)
         return fail(-1, "CFL reduction needs %d partials, the buffer holds %d", nb, capacity);
-    int rc;
-    {
-    TimedScope ts(timed ? kKIcfl : -1); // the per-cell pass (the single-block final reduction is not included)
-    rc = dispatch_nf_d([&](auto NF, auto D) -> int {
+    TimedScope ts(timed ? kKIcfl : -1);
+    const int rc = dispatch_nf_d([&](auto NF, auto D) -> int {
         if (from_cons)
-            hipLaunchKernelGGL((k_icfl<decltype(NF)::value, decltype(D)::value, true>), dim3(nb), dim3(256), 0,
-                               G.stream, f, e, x, dxs[0], dxs[1], dxs[2], dt, G.nint, partials);
+            hipLaunchKernelGGL((k_icfl<decltype(NF)::value, decltype(D)::value, true>), dim3(nb), dim3(kCflThreads), 0,
+                               G.stream, f, e, x, dxs[0], dxs[1], dxs[2], dt, G.nint, partials, G.count, G.result);
         else
-            hipLaunchKernelGGL((k_icfl<decltype(NF)::value, decltype(D)::value, false>), dim3(nb), dim3(256), 0,
-                               G.stream, f, e, x, dxs[0], dxs[1], dxs[2], dt, G.nint, partials);
+            hipLaunchKernelGGL((k_icfl<decltype(NF)::value, decltype(D)::value, false>), dim3(nb), dim3(kCflThreads), 0,
+                               G.stream, f, e, x, dxs[0], dxs[1], dxs[2], dt, G.nint, partials, G.count, G.result);
         HIPCHK(hipGetLastError());
         return 0;
     });
-    }
     if (rc) return rc;
-    hipLaunchKernelGGL(k_reduce_max, dim3(1), dim3(1024), 0, G.stream, partials, nb);
-    HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(out, partials, sizeof(double), hipMemcpyDeviceToHost, G.stream));
     HIPCHK(hipStreamSynchronize(G.stream));
+    *out = *(volatile double *)G.result;
     return 0;
 }
 
@@ -1492,6 +1528,8 @@ int mfc_rhs_finalize(void) {
         G.dir[d] = Dir();
     }
     if (G.partials) (void)hipFree(G.partials);
+    if (G.count) (void)hipFree(G.count);
+    if (G.result) (void)hipHostFree(G.result);
     if (G.scratch_state) (void)hipFree(G.scratch_state);
     if (G.visc_fs) (void)hipFree(G.visc_fs);
     if (G.visc_grad) (void)hipFree(G.visc_grad);
