@@ -139,11 +139,8 @@ struct State {
     double *scratch_state = nullptr; // S*ng doubles, RK3 stage buffer
     bool visc = false;               // any fluid_pp%Re > 0
     ViscParams vp{};
-    double *visc_fs = nullptr;       // (S+2+D) x faces of one direction: HLLC flux, contact velocity, viscous flux
-    long visc_nface = 0;
     bool wrf = false;                // viscous with weno_Re_flux: WENO-reconstructed velocity gradients
     double *visc_grad = nullptr;     // D*D planes of ng: cell-centred velocity gradients (weno_Re_flux)
-    double *visc_fgrad = nullptr;    // D*D planes of visc_nface: their face averages (weno_Re_flux)
 } G;
 
 // ---------------------------------------------------------------------------
@@ -916,8 +913,6 @@ int viscous(int d, const Fields &qin, const Fields &rhs, const SweepArgs &sa) {
     memset(&v, 0, sizeof v);
     v.q = qin;
     v.rhs = rhs;
-    v.fs = G.visc_fs;
-    v.nface = d == 0 ? (long)(G.prm.m + 2) * (G.prm.n + 1) : (long)(G.prm.m + 1) * (G.prm.n + 2);
     v.coef = G.dir[d].coef;
     v.ncell = G.dir[d].s + 2 * G.b + 1;
     v.uniform = G.dir[d].uniform ? 1 : 0;
@@ -937,7 +932,6 @@ int viscous(int d, const Fields &qin, const Fields &rhs, const SweepArgs &sa) {
     v.bc_end = bcs[d][1];
     v.vp = G.vp;
     v.grad = G.visc_grad;
-    v.fgrad = G.visc_fgrad;
     v.ng = G.ng;
     v.wrf = G.wrf ? 1 : 0;
     TimedScope ts(kKViscous);
@@ -975,29 +969,26 @@ int sweeps(const Fields &qin, const Fields &rhs, int rk, const Fields *qbase, co
     if (G.wrf) {
         // cell-centred velocity gradients of the stage input (s_get_viscous,
         // m_rhs.fpp:456-464), before the directions
+        ViscGradArgs g;
+        memset(&g, 0, sizeof g);
+        g.q = qin;
+        g.grad = G.visc_grad;
+        g.eps = G.prm.weno_eps;
+        g.nxg = G.nxg;
+        g.ng = G.ng;
+        g.b = G.b;
+        g.uniform = 1;
         for (int e = 0; e < G.D; ++e) {
-            ViscGradArgs g;
-            memset(&g, 0, sizeof g);
-            g.q = qin;
-            g.grad = G.visc_grad;
-            g.coef = G.dir[e].coef;
-            g.ncell = G.dir[e].s + 2 * G.b + 1;
-            g.inv_dsg = G.dir[e].inv_dsg;
-            g.eps = G.prm.weno_eps;
-            g.nxg = G.nxg;
-            g.ng = G.ng;
-            g.m = G.prm.m;
-            g.n = G.prm.n;
-            g.b = G.b;
-            g.bj = G.prm.n > 0 ? G.b : 0;
-            g.s = G.dir[e].s;
-            g.uniform = G.dir[e].uniform_wide ? 1 : 0;
-            for (int q = 0; q < kNCoef; ++q) g.ucf[q] = G.dir[e].ucf[q];
-            TimedScope ts(kKViscous);
-            if (launch_visc_grad(G.prm.num_fluids, G.D, e, G.prm.weno_order, g, G.stream))
-                return fail(-3, "viscous gradient launch failed (dir %d): %s", e,
-                            hipGetErrorString(hipGetLastError()));
+            g.coef[e] = G.dir[e].coef;
+            g.ncell[e] = G.dir[e].s + 2 * G.b + 1;
+            g.inv_dsg[e] = G.dir[e].inv_dsg;
+            g.s[e] = G.dir[e].s;
+            g.uniform &= G.dir[e].uniform_wide ? 1 : 0;
+            for (int q = 0; q < kNCoef; ++q) g.ucf[e][q] = G.dir[e].ucf[q];
         }
+        TimedScope ts(kKViscous);
+        if (launch_visc_grad(G.prm.num_fluids, G.D, G.prm.weno_order, g, G.stream))
+            return fail(-3, "viscous gradient launch failed: %s", hipGetErrorString(hipGetLastError()));
     }
     // The contracted form spreads an RK stage over its sweeps (out = cb*base
     // + ci*in + cdt*L; the sweeps before the last read the base, the last
@@ -1182,13 +1173,8 @@ int mfc_rhs_init(const mfc_params *prm) {
             }
     G.visc = G.vp.size[0] > 0 || G.vp.size[1] > 0;
     if (G.visc) {
-        G.visc_nface = std::max((long)(prm->m + 2) * (prm->n + 1), (long)(prm->m + 1) * (prm->n + 2));
-        HIPCHK(hipMalloc(&G.visc_fs, sizeof(double) * (G.S + 2 + G.D) * G.visc_nface));
         G.wrf = prm->weno_Re_flux != 0;
-        if (G.wrf) {
-            HIPCHK(hipMalloc(&G.visc_grad, sizeof(double) * G.D * G.D * G.ng));
-            HIPCHK(hipMalloc(&G.visc_fgrad, sizeof(double) * G.D * G.D * G.visc_nface));
-        }
+        if (G.wrf) HIPCHK(hipMalloc(&G.visc_grad, sizeof(double) * G.D * G.D * G.ng));
     }
     G.init = true;
     return 0;
@@ -1531,9 +1517,7 @@ int mfc_rhs_finalize(void) {
     if (G.count) (void)hipFree(G.count);
     if (G.result) (void)hipHostFree(G.result);
     if (G.scratch_state) (void)hipFree(G.scratch_state);
-    if (G.visc_fs) (void)hipFree(G.visc_fs);
     if (G.visc_grad) (void)hipFree(G.visc_grad);
-    if (G.visc_fgrad) (void)hipFree(G.visc_fgrad);
     if (G.own) (void)hipStreamDestroy(G.own);
     G = State();
     return 0;

@@ -11,13 +11,13 @@
 // reconstructed once (both faces), one variable at a time.  The
 // finite-difference gradients come from the primitive velocities (of the
 // tile, and for the x faces' neighbours in y of the conservative field);
-// with weno_Re_flux, gradient planes and their face averages are computed
-// by two passes before the face kernels.  Per face they store the HLLC flux,
-// the contact velocity and the viscous source flux
-// (m_riemann_solvers.fpp:683-902); a finish kernel per direction applies the
-// flux divergence, the alpha*div(u) source and the viscous divergence in the
-// reference's order (m_rhs.fpp:565-652), and in the last direction the RK
-// stage.
+// with weno_Re_flux, gradient planes computed by a pass before the
+// directions are reconstructed in the tile too.  Per face they form the HLLC
+// flux, the contact velocity and the viscous source flux
+// (m_riemann_solvers.fpp:683-902), and then finish the cells between their
+// faces: the flux divergence, the alpha*div(u) source and the viscous
+// divergence in the reference's order (m_rhs.fpp:565-652), and in the last
+// direction the RK stage.
 #include "mfc_viscous.hpp"
 
 namespace mfc {
@@ -143,132 +143,145 @@ __device__ __forceinline__ void fd_averages(const double *gn, const double *gt, 
     }
 }
 
-// The face averages precomputed by k_visc_face_grad (weno_Re_flux).
-template <int D>
-__device__ __forceinline__ void weno_averages(const ViscArgs &a, long t, double *ax, double *ay) {
+// Holds a variable's face states where they are computed: without it the
+// compiler starts every variable's reconstruction before it ends the first.
+__device__ __forceinline__ void pin(double &l, double &r) { asm volatile("" : "+v"(l), "+v"(r)); }
+
+// Finish of one cell, in the reference's order (m_rhs.fpp:565-652): the flux
+// divergence (assigned in the first direction, added after), the alpha*div(u)
+// source, the viscous divergence of momentum and energy; then the rhs store,
+// or the RK stage in the last direction (the sweeps' rk_combine arithmetic).
+// d: lower minus upper face of the S fluxes, dus: upper minus lower contact
+// velocity, dv: lower minus upper face of the viscous fluxes.
+template <int NF, int D>
+__device__ __forceinline__ void visc_finish(const SweepArgs &s, int i, int j, double inv, const double *d, double dus,
+                                            const double *dv) {
+    using Y = Sys<NF, D>;
+    constexpr int S = Y::S;
+    const long go = ghost_off(s, i, j, 0), t = (long)j * (s.m + 1) + i;
+    double r[S];
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-        ax[c] = c < D ? a.fgrad[(long)c * a.nface + t] : 0.0;
-        ay[c] = c < D && D == 2 ? a.fgrad[(long)(D + c) * a.nface + t] : 0.0;
+    for (int v = 0; v < S; ++v) r[v] = s.accumulate ? s.rhs.v[v][t] + inv * d[v] : inv * d[v];
+#pragma unroll
+    for (int k = 0; k < NF; ++k) r[Y::ADV + k] = r[Y::ADV + k] + inv * s.qin.v[Y::ADV + k][go] * dus;
+#pragma unroll
+    for (int v = 0; v <= D; ++v) r[Y::MOM + v] = r[Y::MOM + v] + inv * dv[v];
+    if (s.rk == kRkNone) {
+#pragma unroll
+        for (int v = 0; v < S; ++v) s.rhs.v[v][t] = r[v];
+        return;
+    }
+    // combined and stored per variable (rk_combine's arithmetic; its results in
+    // an array stayed in scratch memory here)
+    switch (s.rk) {
+    case kRkEuler:
+#pragma unroll
+        for (int v = 0; v < S; ++v) s.qout.v[v][go] = s.qbase.v[v][go] + s.dt * r[v];
+        break;
+    case kRk2Final:
+#pragma unroll
+        for (int v = 0; v < S; ++v) s.qout.v[v][go] = (s.qbase.v[v][go] + s.qin.v[v][go] + s.dt * r[v]) / 2.0;
+        break;
+    case kRk3Stage2:
+#pragma unroll
+        for (int v = 0; v < S; ++v) s.qout.v[v][go] = (3.0 * s.qbase.v[v][go] + s.qin.v[v][go] + s.dt * r[v]) / 4.0;
+        break;
+    default:
+#pragma unroll
+        for (int v = 0; v < S; ++v)
+            s.qout.v[v][go] = third(s.qbase.v[v][go] + 2.0 * s.qin.v[v][go] + 2.0 * s.dt * r[v]);
+        break;
     }
 }
 
-// The face record: the HLLC flux (S), the contact velocity and the viscous
-// source flux (D+1), plane p of face t at fs[p * nface + t].
-template <int NF, int D>
-__device__ __forceinline__ void store_face(const ViscArgs &a, long t, const double *flux, double ustar,
-                                           const double *fs) {
-    constexpr int S = Sys<NF, D>::S;
-#pragma unroll
-    for (int v = 0; v < S; ++v) a.fs[(long)v * a.nface + t] = flux[v];
-    a.fs[(long)S * a.nface + t] = ustar;
-#pragma unroll
-    for (int v = 0; v <= D; ++v) a.fs[(long)(S + 1 + v) * a.nface + t] = fs[v];
+// The face average of gradient plane values reconstructed at the upper face of
+// the left cell (R, dqR_prim_d*_n) and the lower face of the right cell (L,
+// dqL_prim_d*_n), with the bc = -4 copies of
+// s_populate_riemann_states_variables_buffers (m_riemann_solvers.fpp:488-608,
+// with the caller's L/R swap), then 5e-1*(R + L) as
+// s_compute_viscous_source_flux averages them (:683-902).
+__device__ __forceinline__ double grad_average(const ViscArgs &a, int f, int s, double R, double L) {
+    if (f == -1 && a.bc_beg == -4) R = L;
+    if (f == s && a.bc_end == -4) L = R;
+    return 5e-1 * (R + L);
 }
 
-// Gradient planes of direction E (weno_Re_flux), one thread per ghosted
-// cell: each velocity component reconstructed along E with WENO over cells
-// [-b+polyn, s+b-polyn] (s_reconstruct_cell_boundary_values_visc,
-// m_viscous.fpp:400-469), then d u_c / d x_E = 1/ds * (vR - vL)
+// Gradient planes of every direction (weno_Re_flux), one thread per ghosted
+// cell: each velocity component reconstructed along direction e with WENO over
+// cells [-b+polyn, s+b-polyn] (s_reconstruct_cell_boundary_values_visc,
+// m_viscous.fpp:400-469), then d u_c / d x_e = 1/ds * (vR - vL)
 // (s_apply_scalar_divergence_theorem, :372-398) over [-b+1, s+b-1].  Cells
 // where the reference reads face values it never wrote, or never writes the
 // gradient, get NaN: their reconstructions reach no face flux the RHS uses.
-template <int NF, int D, int E, int WO, bool UNI>
-__global__ __launch_bounds__(256) void k_visc_grad(ViscGradArgs g) {
+//
+// A block takes kGX x kGY cells and computes the velocities of them and their
+// halos once, into LDS: in a pass per direction with the stencil's velocities
+// per thread, five divisions a component, 1000 x 800 cells took 48 instead of
+// 38 us.
+constexpr int kGX = 32, kGY = 8;
+
+template <int NF, int D, int WO, bool UNI>
+__global__ __launch_bounds__(kGX *kGY) void k_visc_grad(ViscGradArgs g) {
     using Y = Sys<NF, D>;
     constexpr int P = (WO - 1) / 2;
-    const long o = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (o >= g.ng) return;
-    const int i = (int)(o % g.nxg) - g.b;
-    const int j = (int)(o / g.nxg) - g.bj;
-    const int je = E == 0 ? i : j;
-    const bool set = je >= -g.b + P && je <= g.s + g.b - P && je >= -g.b + 1 && je <= g.s + g.b - 1;
-    const long step = E == 0 ? 1 : g.nxg;
-    double cf[kNCoef];
-    if (set) {
+    constexpr int CX = D == 2 ? kGX : kGX * kGY, CY = D == 2 ? kGY : 1; // cells of the tile
+    constexpr int PY = D == 2 ? P : 0;
+    constexpr int HX = CX + 2 * P, HY = CY + 2 * PY;
+    __shared__ double su[D][HY][HX];
+    const int tid = threadIdx.x;
+    const int nyg = D == 2 ? g.s[1] + 1 + 2 * g.b : 1;
+    const int x0 = (int)(blockIdx.x % g.ntile) * CX, y0 = (int)(blockIdx.x / g.ntile) * CY; // ghosted cell counts
+    for (int e = tid; e < HX * HY; e += kGX * kGY) {
+        const int r = e / HX, c = e % HX;
+        const long o = min(max(x0 + c - P, 0), (int)g.nxg - 1) + g.nxg * (long)min(max(y0 + r - PY, 0), nyg - 1);
+        double rho = 0.0;
 #pragma unroll
-        for (int q = 0; q < kNCoef; ++q) cf[q] = UNI ? g.ucf[q] : g.coef[(long)q * g.ncell + (je + g.b)];
+        for (int f = 0; f < NF; ++f) rho = rho + g.q.v[f][o];
+        rho = max_ref(rho, 1e-16);
+#pragma unroll
+        for (int d = 0; d < D; ++d) su[d][r][c] = g.q.v[Y::MOM + d][o] / rho;
     }
-    double st[D][WO];
-    if (set) {
+    __syncthreads();
+    const int tx = tid % CX, ty = tid / CX, xg = x0 + tx, yg = y0 + ty;
+    if (xg >= g.nxg || yg >= nyg) return;
+    const long o = xg + g.nxg * (long)yg;
 #pragma unroll
-        for (int r = 0; r < WO; ++r) {
-            const long oc = o + (r - P) * step;
-            double rho = 0.0;
-#pragma unroll
-            for (int f = 0; f < NF; ++f) rho = rho + g.q.v[f][oc];
-            rho = max_ref(rho, 1e-16);
-#pragma unroll
-            for (int c = 0; c < D; ++c) st[c][r] = g.q.v[Y::MOM + c][oc] / rho;
-        }
-    }
-#pragma unroll
-    for (int c = 0; c < D; ++c) {
-        double val = __builtin_nan("");
+    for (int e = 0; e < D; ++e) {
+        const int i = (e == 0 ? xg : yg) - g.b; // the cell's index along e
+        const bool set = i >= -g.b + P && i <= g.s[e] + g.b - P && i >= -g.b + 1 && i <= g.s[e] + g.b - 1;
+        double cf[kNCoef], inv = 0.0;
         if (set) {
-            double vl, vr;
-            weno_cell<WO, double, true, true>(st[c], cf, g.eps, vl, vr);
-            val = g.inv_dsg[je + g.b] * (vr - vl);
+#pragma unroll
+            for (int q = 0; q < kNCoef; ++q) cf[q] = UNI ? g.ucf[e][q] : g.coef[e][(long)q * g.ncell[e] + (i + g.b)];
+            inv = g.inv_dsg[e][i + g.b];
         }
-        g.grad[(long)(E * D + c) * g.ng + o] = val;
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            double val = __builtin_nan("");
+            if (set) {
+                double st[WO], vl, vr;
+#pragma unroll
+                for (int r = 0; r < WO; ++r)
+                    st[r] = e == 0 ? su[d][ty + PY][tx + r] : su[d][ty + r][tx + P];
+                weno_cell<WO, double, true, true>(st, cf, g.eps, vl, vr);
+                val = inv * (vr - vl);
+            }
+            g.grad[(long)(e * D + d) * g.ng + o] = val;
+        }
     }
 }
 
-// Face averages of the gradients for the faces of direction DIR
-// (weno_Re_flux), one thread per face: each gradient plane reconstructed
-// along DIR (s_reconstruct_cell_boundary_values_visc_deriv,
-// m_viscous.fpp:471-591) at the upper face of the left cell (dqR_prim_d*_n)
-// and the lower face of the right cell (dqL_prim_d*_n), the bc = -4 copies
-// of s_populate_riemann_states_variables_buffers (m_riemann_solvers.fpp:
-// 488-608, with the caller's L/R swap), then 5e-1*(R + L) as
-// s_compute_viscous_source_flux averages them (:683-902).
-template <int NF, int D, int DIR, int WO, bool UNI>
-__global__ __launch_bounds__(256) void k_visc_face_grad(ViscArgs a) {
-    constexpr int P = (WO - 1) / 2;
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= a.nface) return;
-    int x, y, f, s;
-    if constexpr (DIR == 0) {
-        f = (int)(t % (a.m + 2)) - 1;
-        y = (int)(t / (a.m + 2));
-        x = f;
-        s = a.m;
-    } else {
-        x = (int)(t % (a.m + 1));
-        f = (int)(t / (a.m + 1)) - 1;
-        y = f;
-        s = a.n;
-    }
-    const long step = DIR == 0 ? 1 : a.nxg;
-    const long o0 = (long)(x + a.b) + a.nxg * (long)(y + a.bj); // cell f of the face's pair
-    double cf0[kNCoef], cf1[kNCoef];
-    cell_coef<UNI>(a, f, cf0);
-    cell_coef<UNI>(a, f + 1, cf1);
-#pragma unroll
-    for (int pl = 0; pl < D * D; ++pl) {
-        const double *G = a.grad + (long)pl * a.ng;
-        double st[WO], dummy, R, L;
-#pragma unroll
-        for (int r = 0; r < WO; ++r) st[r] = G[o0 + (r - P) * step];
-        weno_cell<WO, double, false, true>(st, cf0, a.eps, dummy, R);
-#pragma unroll
-        for (int r = 0; r < WO; ++r) st[r] = G[o0 + (r + 1 - P) * step];
-        weno_cell<WO, double, true, false>(st, cf1, a.eps, L, dummy);
-        if (f == -1 && a.bc_beg == -4) R = L;
-        if (f == s && a.bc_end == -4) L = R;
-        a.fgrad[(long)pl * a.nface + t] = 5e-1 * (R + L);
-    }
-}
-
-// x faces: one wave per 63 faces f0 .. f0+62 of row y (f0 = -1 + 63*tile).
-// Lane l converts stencil cells into LDS once, then reconstructs both faces
-// of cell c = f0 + l (the smoothness indicators shared, as in the
+// x direction: one wave per 62 cells f0+1 .. f0+62 of row y (f0 = -1 +
+// 62*tile).  Lane l converts stencil cells into LDS once, then reconstructs
+// both faces of cell c = f0 + l (the smoothness indicators shared, as in the
 // cell-parallel sweeps); face f = c takes its right state, the left-face
-// value of cell c+1, from the next lane.  No register cap: the kernel takes
-// 230 VGPRs (2 waves per SIMD) for two fluids in 2D; capped at 4 or 3 waves
-// it spills and is slower.
+// value of cell c+1, from the next lane, and cell f+1 its upper face's fluxes
+// the same way.  Bound by FP64 issue (1000 x 800 cells, two fluids, per-cell
+// coefficients: 2470 vector instructions a wave, 1960 of them FP64).  With the
+// faces' records stored for a finish kernel, and the gradients' face averages
+// by another pass, the direction took 71 + 22 + 40 us instead of 90 together.
 template <int NF, int D, int WO, bool UNI, bool WRF>
-__global__ __launch_bounds__(64) void k_visc_face_x(ViscArgs a, int ntile) {
+__global__ __launch_bounds__(64) void k_visc_x(ViscArgs a, SweepArgs s, int ntile) {
     using Y = Sys<NF, D>;
     constexpr int S = Y::S;
     constexpr int P = (WO - 1) / 2;
@@ -277,7 +290,7 @@ __global__ __launch_bounds__(64) void k_visc_face_x(ViscArgs a, int ntile) {
     const int lane = threadIdx.x;
     const int tile = (int)(blockIdx.x % ntile);
     const int y = (int)(blockIdx.x / ntile);
-    const int f0 = -1 + 63 * tile;
+    const int f0 = -1 + 62 * tile;
     const int hi = a.m + a.b; // last ghost cell
     for (int k = lane; k < NS; k += 64) {
         const int c = min(f0 - P + k, hi);
@@ -293,24 +306,32 @@ __global__ __launch_bounds__(64) void k_visc_face_x(ViscArgs a, int ntile) {
     const int c = min(f0 + lane, hi - P); // this lane's cell (clamped past the last face)
     double cf[kNCoef];
     cell_coef<UNI>(a, c, cf);
-    // one variable at a time (bounded registers); the face states go to LDS
-    // rows only this lane reads back: its upper-face value, and the next
-    // lane's lower-face value
-    __shared__ double sq[2][S][64];
+    // face averages of the gradient planes, reconstructed along x
+    // (s_reconstruct_cell_boundary_values_visc_deriv, m_viscous.fpp:471-591)
+    __shared__ double sg[WRF ? D * D : 1][64]; // rows only this lane reads back
+    if constexpr (WRF) {
+        const long o = goff(a, c, y);
+        const int f = min(f0 + lane, a.m);
 #pragma unroll 1
-    for (int v = 0; v < S; ++v) {
-        double st[WO], vl, vr;
+        for (int pl = 0; pl < D * D; ++pl) {
+            const double *G = a.grad + (long)pl * a.ng + o;
+            double st[WO], vl, vr;
 #pragma unroll
-        for (int r = 0; r < WO; ++r) st[r] = sp[v][lane + r];
-        weno_cell<WO, double, true, true>(st, cf, a.eps, vl, vr);
-        sq[0][v][lane] = vr;
-        sq[1][v][lane] = __shfl_down(vl, 1, 64);
+            for (int r = 0; r < WO; ++r) st[r] = G[r - P];
+            weno_cell<WO, double, true, true>(st, cf, a.eps, vl, vr);
+            sg[pl][lane] = grad_average(a, f, a.m, vr, __shfl_down(vl, 1, 64));
+        }
     }
+    // one variable's registers at a time
     double ql[S], qr[S];
 #pragma unroll
     for (int v = 0; v < S; ++v) {
-        ql[v] = sq[0][v][lane];
-        qr[v] = sq[1][v][lane];
+        double st[WO], vl;
+#pragma unroll
+        for (int r = 0; r < WO; ++r) st[r] = sp[v][lane + r];
+        weno_cell<WO, double, true, true>(st, cf, a.eps, vl, ql[v]);
+        qr[v] = __shfl_down(vl, 1, 64);
+        pin(ql[v], qr[v]);
     }
     // velocities of rows y-1 and y+1 of this lane's cell, then of the next
     // lane's (2D transverse gradients)
@@ -337,8 +358,7 @@ __global__ __launch_bounds__(64) void k_visc_face_x(ViscArgs a, int ntile) {
             gt[d] = 25e-2 * sum;
         }
     }
-    const int f = f0 + lane;
-    if (lane == 63 || f > a.m) return;
+    const int f = min(f0 + lane, a.m); // (clamped past the last face)
     if (f == -1 && a.bc_beg == -4) {
 #pragma unroll
         for (int v = 0; v < S; ++v) ql[v] = qr[v];
@@ -347,10 +367,13 @@ __global__ __launch_bounds__(64) void k_visc_face_x(ViscArgs a, int ntile) {
 #pragma unroll
         for (int v = 0; v < S; ++v) qr[v] = ql[v];
     }
-    const long t = (long)y * (a.m + 2) + (f + 1);
     double ax[2], ay[2];
     if constexpr (WRF) {
-        weno_averages<D>(a, t, ax, ay);
+#pragma unroll
+        for (int d = 0; d < 2; ++d) {
+            ax[d] = d < D ? sg[d][lane] : 0.0;
+            ay[d] = d < D && D == 2 ? sg[D + d][lane] : 0.0;
+        }
     } else {
         // one-sided x differences across the face (dqR_prim_dx_n(1) at x)
         double gxn[2] = {0.0, 0.0};
@@ -361,49 +384,84 @@ __global__ __launch_bounds__(64) void k_visc_face_x(ViscArgs a, int ntile) {
     }
     double flux[S], ustar, fs[D + 1];
     face_flux<NF, D, 0>(a, ql, qr, ax, ay, flux, ustar, fs);
-    store_face<NF, D>(a, t, flux, ustar, fs);
+    const double dus = __shfl_down(ustar, 1, 64) - ustar;
+#pragma unroll
+    for (int v = 0; v < S; ++v) flux[v] = flux[v] - __shfl_down(flux[v], 1, 64);
+#pragma unroll
+    for (int v = 0; v <= D; ++v) fs[v] = fs[v] - __shfl_down(fs[v], 1, 64);
+    const int i = f0 + lane + 1;
+    if (lane < 62 && i <= a.m) visc_finish<NF, D>(s, i, y, a.inv_ds[i], flux, dus, fs);
 }
 
-// y faces (2D), cell-parallel on an LDS tile: a 256-thread block covers
-// kYC x-columns by kYK cells along y, the K lanes of a column consecutive
-// in the wave.  The primitive stencil rows of the tile (with one x-halo
-// column on each side, for the transverse velocity differences) are
-// converted once into LDS; thread (column, c) reconstructs both faces of
-// cell f0+c one variable at a time (the WENO of the sweeps), its upper-face
-// value and the next lane's lower-face value go to LDS as the states of
-// face f0+c+1/2, and after a barrier the first K-1 lanes of each column
-// solve their faces (HLLC, face Reynolds numbers, gradients, viscous flux)
-// and store the face records.  Each cell is converted and reconstructed
-// once, with the per-variable reconstruction bounded to one variable's
-// registers (a thread marching along y with the stencil window in registers
-// held 256 VGPRs and 72 AGPRs: one wave per SIMD).
+// y direction (2D), cell-parallel on an LDS tile: a block covers kYC
+// x-columns by kYK cells along y, the K lanes of a column consecutive in the
+// wave.  The primitive stencil rows of the tile (for finite-difference
+// gradients with one x-halo column on each side) are converted once into LDS;
+// thread (column, c) reconstructs both faces of cell f0+c one variable at a
+// time (the WENO of the sweeps) and takes the state above its upper face from
+// the next lane, the first K-1 lanes of each column solve their faces (HLLC,
+// face Reynolds numbers, gradients, viscous flux), and after the faces' fluxes
+// have replaced the tile in LDS the K-2 cells between them are finished with
+// the threads along x.  (A thread marching along y with the stencil window in
+// registers held 256 VGPRs and 72 AGPRs: one wave per SIMD.)  As in x, one
+// kernel instead of three: 1000 x 800 cells, two fluids, 110 instead of 80 +
+// 48 + 37 us.  The face states stay in registers: in LDS they halved the
+// blocks per CU (136 us).  32 rows a tile are level with 16.
 constexpr int kYC = 16; // x-columns per tile
-constexpr int kYK = 16; // cells per column (faces: kYK - 1)
+constexpr int kYK = 16; // cells per column (faces: kYK - 1, finished cells: kYK - 2)
 
 template <int NF, int WO, bool UNI, bool WRF>
-__global__ __launch_bounds__(kYC *kYK) void k_visc_face_yc(ViscArgs a, int nxb) {
+__global__ __launch_bounds__(kYC *kYK) void k_visc_y(ViscArgs a, SweepArgs s, int nxb) {
     constexpr int D = 2;
     using Y = Sys<NF, D>;
     constexpr int S = Y::S;
     constexpr int P = (WO - 1) / 2;
-    constexpr int R = kYK + 2 * P; // stencil rows f0-P .. f0+K-1+P
-    constexpr int XC = kYC + 2;     // columns x0-1 .. x0+C
+    constexpr int R = kYK + 2 * P;  // stencil rows f0-P .. f0+K-1+P
+    constexpr int XH = WRF ? 0 : 1; // x-halo columns on each side
+    constexpr int XC = kYC + 2 * XH;
     // stencil rows of each column contiguous (odd pitch R + 1): the lanes of
     // a column read consecutive entries
-    __shared__ double sp[S][XC][R + 1];
-    // face f0+c+1/2 of column col: left state (upper face of cell f0+c) and
-    // right state (lower face of cell f0+c+1), c fastest (the lanes of a
-    // column are consecutive: conflict-free LDS access)
-    __shared__ double sL[S][kYC][kYK];
-    __shared__ double sR[S][kYC][kYK];
+    using Tile = double[XC][R + 1];
+    // then the S fluxes, the contact velocity and the viscous fluxes of face
+    // f0+c+1/2 of column col, with an odd pitch for the finish along x
+    using Face = double[kYC][kYK + 1];
+    constexpr int NT = S * sizeof(Tile) / 8, NF_ = (S + 2 + D) * sizeof(Face) / 8;
+    __shared__ double sh[NT > NF_ ? NT : NF_];
+    Tile *sp = reinterpret_cast<Tile *>(sh);
+    Face *sf = reinterpret_cast<Face *>(sh);
     const int tid = threadIdx.x;
     const int col = tid / kYK, c = tid % kYK;
     const int x0 = (int)(blockIdx.x % nxb) * kYC;
-    const int f0 = -1 + (kYK - 1) * (int)(blockIdx.x / nxb);
+    const int f0 = -1 + (kYK - 2) * (int)(blockIdx.x / nxb);
     const int hx = a.m + a.b, hy = a.n + a.b; // last ghost cells
+    const int x = x0 + col;
+    const int f = f0 + c; // this lane's cell, and the face above it
+    double cf[kNCoef];
+    cell_coef<UNI>(a, min(f, hy - P), cf);
+    // face averages of the gradient planes, reconstructed along y
+    __shared__ double sg[WRF ? D * D : 1][kYC * kYK]; // slots only their own thread reads back
+    if constexpr (WRF) {
+        static_assert(S >= D * D, "the gradient planes fit in the tile");
+        for (int e = tid; e < R * kYC; e += kYC * kYK) {
+            const int r = e / kYC, xc = e % kYC;
+            const long o = goff(a, min(x0 + xc, hx), min(f0 - P + r, hy));
+#pragma unroll
+            for (int pl = 0; pl < D * D; ++pl) sp[pl][xc][r] = a.grad[(long)pl * a.ng + o];
+        }
+        __syncthreads();
+#pragma unroll 1
+        for (int pl = 0; pl < D * D; ++pl) {
+            double st[WO], vl, vr;
+#pragma unroll
+            for (int r = 0; r < WO; ++r) st[r] = sp[pl][col][c + r];
+            weno_cell<WO, double, true, true>(st, cf, a.eps, vl, vr);
+            sg[pl][tid] = grad_average(a, f, a.n, vr, __shfl_down(vl, 1, 64));
+        }
+        __syncthreads();
+    }
     for (int e = tid; e < R * XC; e += kYC * kYK) {
         const int r = e / XC, xc = e % XC;
-        const long o = goff(a, min(x0 - 1 + xc, hx), min(f0 - P + r, hy));
+        const long o = goff(a, min(x0 - XH + xc, hx), min(f0 - P + r, hy));
         double cv[S], pv[S];
 #pragma unroll
         for (int v = 0; v < S; ++v) cv[v] = a.q.v[v][o];
@@ -412,163 +470,107 @@ __global__ __launch_bounds__(kYC *kYK) void k_visc_face_yc(ViscArgs a, int nxb) 
         for (int v = 0; v < S; ++v) sp[v][xc][r] = pv[v];
     }
     __syncthreads();
-    const int x = x0 + col;
-    const int cy = f0 + c; // this lane's cell
-    double cf[kNCoef];
-    cell_coef<UNI>(a, min(cy, hy - P), cf);
-#pragma unroll 1
-    for (int v = 0; v < S; ++v) {
-        double st[WO], vl, vr;
-#pragma unroll
-        for (int r = 0; r < WO; ++r) st[r] = sp[v][col + 1][c + r];
-        weno_cell<WO, double, true, true>(st, cf, a.eps, vl, vr);
-        sL[v][col][c] = vr;
-        // lane c+1 of the same column holds cell f0+c+1 (the last lane's value
-        // is not used)
-        sR[v][col][c] = __shfl_down(vl, 1, 64);
-    }
-    __syncthreads();
-    const int f = cy;
-    if (c == kYK - 1 || x > a.m || f > a.n) return;
+    // one variable's registers at a time; lane c+1 of the same column holds
+    // cell f0+c+1 (the last lane's value is not used)
     double ql[S], qr[S];
 #pragma unroll
     for (int v = 0; v < S; ++v) {
-        ql[v] = sL[v][col][c];
-        qr[v] = sR[v][col][c];
-    }
-    if (f == -1 && a.bc_beg == -4) {
+        double st[WO], vl;
 #pragma unroll
-        for (int v = 0; v < S; ++v) ql[v] = qr[v];
+        for (int r = 0; r < WO; ++r) st[r] = sp[v][col + XH][c + r];
+        weno_cell<WO, double, true, true>(st, cf, a.eps, vl, ql[v]);
+        qr[v] = __shfl_down(vl, 1, 64);
+        pin(ql[v], qr[v]);
     }
-    if (f == a.n && a.bc_end == -4) {
-#pragma unroll
-        for (int v = 0; v < S; ++v) qr[v] = ql[v];
-    }
-    const long t = (long)(f + 1) * (a.m + 1) + x;
-    double ax[2], ay[2];
-    if constexpr (WRF) {
-        weno_averages<D>(a, t, ax, ay);
-    } else {
-        // velocities of cells (x-1 .. x+1, f) and (x-1 .. x+1, f+1)
-        const int r0 = c + P, r1 = c + P + 1;
-        const double dyf = a.ccy[f + 1 + a.b] - a.ccy[f + a.b];
-        const double dxm = a.ccx[x + a.b] - a.ccx[x - 1 + a.b], dxp = a.ccx[x + 1 + a.b] - a.ccx[x + a.b];
-        double gxn[2], gt[2];
-#pragma unroll
-        for (int d = 0; d < 2; ++d) {
-            const double uo = sp[Y::MOM + d][col + 1][r0], uw = sp[Y::MOM + d][col][r0], ue = sp[Y::MOM + d][col + 2][r0];
-            const double no = sp[Y::MOM + d][col + 1][r1], nw = sp[Y::MOM + d][col][r1], ne = sp[Y::MOM + d][col + 2][r1];
-            gxn[d] = (no - uo) / dyf;
-            // four-point average of the one-sided x differences of rows f+1
-            // and f (dqR_prim_dx_n(2) at f, m_viscous.fpp:285-315)
-            const double sum = (no - nw) / dxm + (ne - no) / dxp + (uo - uw) / dxm + (ue - uo) / dxp;
-            gt[d] = 25e-2 * sum;
-        }
-        fd_averages<D, 1>(gxn, gt, ax, ay);
-    }
+    const bool face = c < kYK - 1 && x <= a.m && f <= a.n;
     double flux[S], ustar, fs[D + 1];
-    face_flux<NF, D, 1>(a, ql, qr, ax, ay, flux, ustar, fs);
-    store_face<NF, D>(a, t, flux, ustar, fs);
-}
-
-// Finish of one direction for every interior cell, in the reference's
-// order (m_rhs.fpp:565-652): the flux divergence (assigned in the first
-// direction, added after), the alpha*div(u) source, the viscous divergence
-// of momentum and energy; then the rhs store, or the RK stage in the last
-// direction (the sweeps' finish_cell and rk_combine arithmetic).
-template <int NF, int D, int DIR>
-__global__ __launch_bounds__(256) void k_visc_finish(ViscArgs a, SweepArgs s, long nint) {
-    using Y = Sys<NF, D>;
-    constexpr int S = Y::S;
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nint) return;
-    const int i = (int)(t % (a.m + 1));
-    const int j = (int)(t / (a.m + 1));
-    long fl, fr;
-    double inv;
-    if constexpr (DIR == 0) {
-        fl = (long)j * (a.m + 2) + i; // face i-1/2 is stored at (i-1)+1
-        fr = fl + 1;
-        inv = a.inv_ds[i];
-    } else {
-        fl = (long)j * (a.m + 1) + i;
-        fr = fl + (a.m + 1);
-        inv = a.inv_ds[j];
+    if (face) {
+        if (f == -1 && a.bc_beg == -4) {
+#pragma unroll
+            for (int v = 0; v < S; ++v) ql[v] = qr[v];
+        }
+        if (f == a.n && a.bc_end == -4) {
+#pragma unroll
+            for (int v = 0; v < S; ++v) qr[v] = ql[v];
+        }
+        double ax[2], ay[2];
+        if constexpr (WRF) {
+#pragma unroll
+            for (int d = 0; d < 2; ++d) ax[d] = sg[d][tid], ay[d] = sg[D + d][tid];
+        } else {
+            // velocities of cells (x-1 .. x+1, f) and (x-1 .. x+1, f+1)
+            const int r0 = c + P, r1 = c + P + 1;
+            const double dyf = a.ccy[f + 1 + a.b] - a.ccy[f + a.b];
+            const double dxm = a.ccx[x + a.b] - a.ccx[x - 1 + a.b], dxp = a.ccx[x + 1 + a.b] - a.ccx[x + a.b];
+            double gxn[2], gt[2];
+#pragma unroll
+            for (int d = 0; d < 2; ++d) {
+                const double(*u)[R + 1] = &sp[Y::MOM + d][col];
+                const double uo = u[1][r0], uw = u[0][r0], ue = u[2 * XH][r0];
+                const double no = u[1][r1], nw = u[0][r1], ne = u[2 * XH][r1];
+                gxn[d] = (no - uo) / dyf;
+                // four-point average of the one-sided x differences of rows f+1
+                // and f (dqR_prim_dx_n(2) at f, m_viscous.fpp:285-315)
+                const double sum = (no - nw) / dxm + (ne - no) / dxp + (uo - uw) / dxm + (ue - uo) / dxp;
+                gt[d] = 25e-2 * sum;
+            }
+            fd_averages<D, 1>(gxn, gt, ax, ay);
+        }
+        face_flux<NF, D, 1>(a, ql, qr, ax, ay, flux, ustar, fs);
     }
-    const long go = ghost_off(s, i, j, 0);
-    auto F = [&](int p, long f) { return a.fs[(long)p * a.nface + f]; };
-    double r[S];
+    __syncthreads();
+    if (face) {
 #pragma unroll
-    for (int v = 0; v < S; ++v) {
-        const double df = F(v, fl) - F(v, fr);
-        r[v] = s.accumulate ? s.rhs.v[v][t] + inv * df : inv * df;
+        for (int v = 0; v < S; ++v) sf[v][col][c] = flux[v];
+        sf[S][col][c] = ustar;
+#pragma unroll
+        for (int v = 0; v <= D; ++v) sf[S + 1 + v][col][c] = fs[v];
     }
-    const double dus = F(S, fr) - F(S, fl);
+    __syncthreads();
+    const int fx = tid % kYC, r = tid / kYC, i = x0 + fx, j = f0 + 1 + r;
+    if (r >= kYK - 2 || i > a.m || j > a.n) return;
+    double d[S], dv[D + 1];
 #pragma unroll
-    for (int k = 0; k < NF; ++k) r[Y::ADV + k] = r[Y::ADV + k] + inv * s.qin.v[Y::ADV + k][go] * dus;
+    for (int v = 0; v < S; ++v) d[v] = sf[v][fx][r] - sf[v][fx][r + 1];
 #pragma unroll
-    for (int v = 0; v <= D; ++v) r[Y::MOM + v] = r[Y::MOM + v] + inv * (F(S + 1 + v, fl) - F(S + 1 + v, fr));
-    if (s.rk == kRkNone) {
-#pragma unroll
-        for (int v = 0; v < S; ++v) s.rhs.v[v][t] = r[v];
-        return;
-    }
-    FinishIn<S> fin;
-    double o[S];
-#pragma unroll
-    for (int v = 0; v < S; ++v) {
-        fin.base[v] = s.qbase.v[v][go];
-        fin.in[v] = s.qin.v[v][go];
-    }
-    rk_combine<S>(s, fin, r, o);
-#pragma unroll
-    for (int v = 0; v < S; ++v) s.qout.v[v][go] = o[v];
+    for (int v = 0; v <= D; ++v) dv[v] = sf[S + 1 + v][fx][r] - sf[S + 1 + v][fx][r + 1];
+    visc_finish<NF, D>(s, i, j, a.inv_ds[j], d, sf[S][fx][r + 1] - sf[S][fx][r], dv);
 }
 
 template <int NF, int D, int DIR, int WO, bool UNI, bool WRF>
-void launch_face_u(const ViscArgs &a, hipStream_t st) {
+void launch_dir_u(const ViscArgs &a, const SweepArgs &sa, hipStream_t st) {
     if constexpr (DIR == 0) {
-        const int ntile = (a.m + 2 + 62) / 63;
-        hipLaunchKernelGGL((k_visc_face_x<NF, D, WO, UNI, WRF>), dim3((unsigned)((long)ntile * (a.n + 1))), dim3(64),
-                           0, st, a, ntile);
+        const int ntile = (a.m + 1 + 61) / 62;
+        hipLaunchKernelGGL((k_visc_x<NF, D, WO, UNI, WRF>), dim3((unsigned)((long)ntile * (a.n + 1))), dim3(64), 0, st,
+                           a, sa, ntile);
     } else {
         const int nxb = (a.m + 1 + kYC - 1) / kYC;
-        const int ntile = (a.n + 2 + kYK - 2) / (kYK - 1); // faces -1 .. n in tiles of kYK - 1
-        hipLaunchKernelGGL((k_visc_face_yc<NF, WO, UNI, WRF>), dim3((unsigned)((long)nxb * ntile)),
-                           dim3(kYC * kYK), 0, st, a, nxb);
+        const int ntile = (a.n + 1 + kYK - 3) / (kYK - 2);
+        hipLaunchKernelGGL((k_visc_y<NF, WO, UNI, WRF>), dim3((unsigned)((long)nxb * ntile)), dim3(kYC * kYK), 0, st,
+                           a, sa, nxb);
     }
 }
 
 template <int NF, int D, int DIR, int WO>
-void launch_face(const ViscArgs &a, hipStream_t st) {
+int launch_order(const ViscArgs &a, const SweepArgs &sa, hipStream_t st) {
     if (a.wrf) {
-        const dim3 grid((unsigned)((a.nface + 255) / 256));
-        if (a.uniform) {
-            hipLaunchKernelGGL((k_visc_face_grad<NF, D, DIR, WO, true>), grid, dim3(256), 0, st, a);
-            launch_face_u<NF, D, DIR, WO, true, true>(a, st);
-        } else {
-            hipLaunchKernelGGL((k_visc_face_grad<NF, D, DIR, WO, false>), grid, dim3(256), 0, st, a);
-            launch_face_u<NF, D, DIR, WO, false, true>(a, st);
-        }
+        if (a.uniform) launch_dir_u<NF, D, DIR, WO, true, true>(a, sa, st);
+        else launch_dir_u<NF, D, DIR, WO, false, true>(a, sa, st);
     } else {
-        if (a.uniform) launch_face_u<NF, D, DIR, WO, true, false>(a, st);
-        else launch_face_u<NF, D, DIR, WO, false, false>(a, st);
+        if (a.uniform) launch_dir_u<NF, D, DIR, WO, true, false>(a, sa, st);
+        else launch_dir_u<NF, D, DIR, WO, false, false>(a, sa, st);
     }
+    return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 template <int NF, int D, int DIR>
 int launch_dir(int weno_order, const ViscArgs &a, const SweepArgs &sa, hipStream_t st) {
     switch (weno_order) {
-    case 1: launch_face<NF, D, DIR, 1>(a, st); break;
-    case 3: launch_face<NF, D, DIR, 3>(a, st); break;
-    case 5: launch_face<NF, D, DIR, 5>(a, st); break;
+    case 1: return launch_order<NF, D, DIR, 1>(a, sa, st);
+    case 3: return launch_order<NF, D, DIR, 3>(a, sa, st);
+    case 5: return launch_order<NF, D, DIR, 5>(a, sa, st);
     default: return -1;
     }
-    if (hipGetLastError() != hipSuccess) return -1;
-    const long nint = (long)(a.m + 1) * (a.n + 1);
-    hipLaunchKernelGGL((k_visc_finish<NF, D, DIR>), dim3((unsigned)((nint + 255) / 256)), dim3(256), 0, st, a, sa,
-                       nint);
-    return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 template <int NF>
@@ -579,19 +581,22 @@ int launch_nf(int D, int dir, int weno_order, const ViscArgs &a, const SweepArgs
     return -1;
 }
 
-template <int NF, int D, int E>
-int launch_grad_e(int weno_order, const ViscGradArgs &g, hipStream_t st) {
-    const dim3 grid((unsigned)((g.ng + 255) / 256));
+template <int NF, int D>
+int launch_grad(int weno_order, ViscGradArgs g, hipStream_t st) {
+    const int cx = D == 2 ? kGX : kGX * kGY, cy = D == 2 ? kGY : 1;
+    const int nyg = D == 2 ? g.s[1] + 1 + 2 * g.b : 1;
+    g.ntile = (int)((g.nxg + cx - 1) / cx);
+    const dim3 grid((unsigned)((long)g.ntile * ((nyg + cy - 1) / cy))), block(kGX * kGY);
     const bool u = g.uniform != 0;
     switch (weno_order) {
-    case 1: hipLaunchKernelGGL((k_visc_grad<NF, D, E, 1, false>), grid, dim3(256), 0, st, g); break;
+    case 1: hipLaunchKernelGGL((k_visc_grad<NF, D, 1, false>), grid, block, 0, st, g); break;
     case 3:
-        if (u) hipLaunchKernelGGL((k_visc_grad<NF, D, E, 3, true>), grid, dim3(256), 0, st, g);
-        else hipLaunchKernelGGL((k_visc_grad<NF, D, E, 3, false>), grid, dim3(256), 0, st, g);
+        if (u) hipLaunchKernelGGL((k_visc_grad<NF, D, 3, true>), grid, block, 0, st, g);
+        else hipLaunchKernelGGL((k_visc_grad<NF, D, 3, false>), grid, block, 0, st, g);
         break;
     case 5:
-        if (u) hipLaunchKernelGGL((k_visc_grad<NF, D, E, 5, true>), grid, dim3(256), 0, st, g);
-        else hipLaunchKernelGGL((k_visc_grad<NF, D, E, 5, false>), grid, dim3(256), 0, st, g);
+        if (u) hipLaunchKernelGGL((k_visc_grad<NF, D, 5, true>), grid, block, 0, st, g);
+        else hipLaunchKernelGGL((k_visc_grad<NF, D, 5, false>), grid, block, 0, st, g);
         break;
     default: return -1;
     }
@@ -599,21 +604,20 @@ int launch_grad_e(int weno_order, const ViscGradArgs &g, hipStream_t st) {
 }
 
 template <int NF>
-int launch_grad_nf(int D, int e, int weno_order, const ViscGradArgs &g, hipStream_t st) {
-    if (D == 1 && e == 0) return launch_grad_e<NF, 1, 0>(weno_order, g, st);
-    if (D == 2 && e == 0) return launch_grad_e<NF, 2, 0>(weno_order, g, st);
-    if (D == 2 && e == 1) return launch_grad_e<NF, 2, 1>(weno_order, g, st);
+int launch_grad_nf(int D, int weno_order, const ViscGradArgs &g, hipStream_t st) {
+    if (D == 1) return launch_grad<NF, 1>(weno_order, g, st);
+    if (D == 2) return launch_grad<NF, 2>(weno_order, g, st);
     return -1;
 }
 
 } // namespace
 
-int launch_visc_grad(int nf, int D, int e, int weno_order, const ViscGradArgs &g, hipStream_t st) {
+int launch_visc_grad(int nf, int D, int weno_order, const ViscGradArgs &g, hipStream_t st) {
     switch (nf) {
-    case 1: return launch_grad_nf<1>(D, e, weno_order, g, st);
-    case 2: return launch_grad_nf<2>(D, e, weno_order, g, st);
-    case 3: return launch_grad_nf<3>(D, e, weno_order, g, st);
-    case 4: return launch_grad_nf<4>(D, e, weno_order, g, st);
+    case 1: return launch_grad_nf<1>(D, weno_order, g, st);
+    case 2: return launch_grad_nf<2>(D, weno_order, g, st);
+    case 3: return launch_grad_nf<3>(D, weno_order, g, st);
+    case 4: return launch_grad_nf<4>(D, weno_order, g, st);
     default: return -1;
     }
 }

@@ -23,8 +23,6 @@ struct ViscParams {
 struct ViscArgs {
     Fields q;             // ghost-filled conservative stage input
     Fields rhs;           // interior rhs the divergence is added to
-    double *fs;           // face records, S+2+D planes of nface doubles (HLLC flux, contact velocity, viscous flux)
-    long nface;
     const double *coef;   // WENO coefficients of the sweep direction, 27 planes of ncell
     long ncell;
     int uniform;          // every reconstructed cell has the coefficients ucf (bit for bit)
@@ -37,39 +35,37 @@ struct ViscArgs {
     int m, n, b, bj;
     int bc_beg, bc_end;   // of the sweep direction
     ViscParams vp;
-    // weno_Re_flux: cell-centred velocity gradients, 2*D planes of ng doubles
-    // (plane e*D + c: d u_c / d x_e over the ghosted grid), and their face
-    // averages in the sweep direction, 2*D planes of nface doubles (same
-    // order, face t as in the face record)
+    // weno_Re_flux: cell-centred velocity gradients, D*D planes of ng doubles
+    // (plane e*D + c: d u_c / d x_e over the ghosted grid)
     const double *grad;
-    double *fgrad;
     long ng;
     int wrf;
 };
 
-// Velocity gradients along direction e (weno_Re_flux): the WENO face values
-// of each velocity component along e and the divergence theorem.
+// Velocity gradients (weno_Re_flux): the WENO face values of each velocity
+// component along each direction e and the divergence theorem.
 struct ViscGradArgs {
-    Fields q;               // ghost-filled conservative stage input
-    double *grad;           // the gradient planes (ViscArgs::grad)
-    const double *coef;     // WENO coefficients of direction e, 27 planes of ncell
-    long ncell;
-    const double *inv_dsg;  // 1/ds(i) of direction e over the ghosted range, i = -b..s+b at i+b
+    Fields q;                  // ghost-filled conservative stage input
+    double *grad;              // the gradient planes (ViscArgs::grad)
+    const double *coef[2];     // WENO coefficients of direction e, 27 planes of ncell[e]
+    long ncell[2];
+    const double *inv_dsg[2];  // 1/ds(i) of direction e over the ghosted range, i = -b..s+b at i+b
     double eps;
     long nxg, ng;
-    int m, n, b, bj, s;     // s: last interior index along e
-    int uniform;            // every cell the pass reconstructs has the coefficients ucf (bit for bit)
-    double ucf[kNCoef];
+    int b, s[2];               // s[e]: last interior index along e
+    int ntile;                 // tiles along x
+    int uniform;               // every cell reconstructed along e has the coefficients ucf[e] (bit for bit)
+    double ucf[2][kNCoef];
 };
 
-// Direction dir of a viscous RHS evaluation: the face records, then the
-// finish, which assigns (sa.accumulate = 0) or adds to sa.rhs, or applies
-// the RK stage sa.rk from sa.qbase and sa.qin into sa.qout.
+// Direction dir of a viscous RHS evaluation: the fluxes of its faces, and the
+// cells' finish, which assigns (sa.accumulate = 0) or adds to sa.rhs, or
+// applies the RK stage sa.rk from sa.qbase and sa.qin into sa.qout.
 int launch_viscous(int nf, int D, int dir, int weno_order, const ViscArgs &a, const SweepArgs &sa,
                    hipStream_t stream);
 
-// The gradient planes of direction e (weno_Re_flux), before the directions
-// of a viscous RHS evaluation.
-int launch_visc_grad(int nf, int D, int e, int weno_order, const ViscGradArgs &g, hipStream_t stream);
+// The gradient planes (weno_Re_flux), before the directions of a viscous RHS
+// evaluation.
+int launch_visc_grad(int nf, int D, int weno_order, const ViscGradArgs &g, hipStream_t stream);
 
 } // namespace mfc
