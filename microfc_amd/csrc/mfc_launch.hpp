@@ -4,12 +4,14 @@
 #pragma once
 
 #include "mfc_march.hpp"
+#include "mfc_stage.hpp"
 #include "mfc_sweep.hpp"
 
 namespace mfc {
 
 struct SweepLaunch {
-    int dir;       // 0, 1, 2; 3: the fused x and y sweep (k_sweep_xy); 4: the x and y march; 5: the z march
+    int dir;       // 0, 1, 2; 3: the fused x and y sweep (k_sweep_xy); 4: the x and y march; 5: the z march;
+                   // 6: an RK stage in one kernel (k_stage)
     int num_dims;  // 1..3
     int weno_order;
     int precision; // MFC_PREC_*
@@ -31,6 +33,9 @@ int launch_sweep(const SweepLaunch &L, const SweepArgs &a, hipStream_t st);
             else return -1;                                                                             \
         } else if (dir == 5) {                                                                          \
             if constexpr (NF <= kMarchMaxFluids && D == 3 && WO == 5 && !ML) hipLaunchKernelGGL((k_march<NF, 3, 2, R, false, UNI>), grid, dim3(64), 0, st, a); \
+            else return -1;                                                                             \
+        } else if (dir == 6) {                                                                          \
+            if constexpr (NF <= kXyMaxFluids && D <= 2 && WO == 5 && !ML && sizeof(R) == 8) hipLaunchKernelGGL((k_stage<NF, D, UNI>), grid, dim3(stage_threads(NF, D)), 0, st, a); \
             else return -1;                                                                             \
         } else if (dir == 3) {                                                                          \
             if constexpr (NF <= kXyMaxFluids && D >= 2 && WO == 5 && !ML && UNI) {                      \

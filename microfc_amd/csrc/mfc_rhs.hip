@@ -344,22 +344,6 @@ __device__ __forceinline__ long box_off(const Box &x, int i, int j, int k) {
     return (long)(i + x.b) + x.nxg * ((long)(j + x.bj) + x.nyg * (long)(k + x.bk));
 }
 
-// Source index of a ghost coordinate for one direction's boundary condition
-// (m_rhs.fpp:692-905): <= -3 extrapolation, -2 reflection, -1 periodic.
-__device__ __forceinline__ int bc_source(int bcb, int bce, int s, int i, bool &flip) {
-    if (i < 0) {
-        if (bcb <= -3) return 0;
-        if (bcb == -2) { flip = !flip; return -i - 1; }
-        return s + 1 + i;
-    }
-    if (i > s) {
-        if (bce <= -3) return s;
-        if (bce == -2) { flip = !flip; return 2 * s + 1 - i; }
-        return i - (s + 1);
-    }
-    return i;
-}
-
 // Ghost fill.  The reference fills x ghosts for interior rows, then y ghosts
 // over all x, then z ghosts over all x and y, so a corner holds the interior
 // cell reached by applying each direction's map in turn, with the momentum
@@ -868,15 +852,40 @@ bool marches(int d) {
                0.85 * a.ntile * (d == 4 ? kMarchCellsXY : kMarchCellsZ);
 }
 
+// Arguments of k_stage.
+SweepArgs stage_args() {
+    SweepArgs a = G.D == 2 ? xy_args() : sweep_args(0);
+    if (G.D == 2) {
+        a.coef2 = G.dir[1].coef;
+        a.ncell2 = G.dir[1].s + 2 * G.b + 1;
+        a.uniform = G.dir[0].uniform && G.dir[1].uniform;
+    }
+    a.ntile = (G.prm.m + stage_cells_x(G.D)) / stage_cells_x(G.D);
+    a.nblocks = (long)a.ntile * ((G.prm.n + stage_cells_y(G.D)) / stage_cells_y(G.D));
+    return a;
+}
+
+// Whether an RK stage runs as one kernel (k_stage).  In 2D as long as every
+// block has a compute unit of its own: RK3 step on 256 x 160 cells (256
+// blocks) 66.5 -> 48.1 us, contracted 45.5 -> 38.5 us, but on 256 x 170 cells
+// 66.2 -> 74.3 us.  In 1D blocks share compute units: 1000 cells 29.1 -> 24.3
+// us, 100000 cells 34.9 -> 32.5 us and contracted level, 28.3 and 28.0 us.
+constexpr long kStageBlocks2D = 256, kStageBlocks1D = 1600;
+bool stage_in_one() {
+    return G.D <= 2 && !G.visc && G.prm.weno_order == 5 && G.prm.num_fluids <= kXyMaxFluids &&
+           (G.prm.precision == MFC_PREC_FP64 || G.prm.precision == MFC_PREC_FP64_FAST) &&
+           stage_args().nblocks <= (G.D == 2 ? kStageBlocks2D : kStageBlocks1D);
+}
+
 // d = 0, 1, 2: one direction; d = 3: the fused x and y sweep; d = 4, 5: the
-// marches.
+// marches; d = 6: an RK stage in one kernel.
 int sweep(int d, SweepArgs &a) {
     SweepLaunch L{d, G.D, G.prm.weno_order, G.prm.precision};
     if (G.prm.precision == MFC_PREC_FP32_LEARNED) {
         a.mlp = mlp_frags();
         if (!a.mlp) return fail(-4, "learned weights requested but mfc_mlp_init has not been called");
     }
-    TimedScope ts(d == 3 || d == 4 ? kKSweepXY : d == 5 ? kKSweepZ : kKSweepX + d);
+    TimedScope ts(d == 3 || d == 4 ? kKSweepXY : d == 5 ? kKSweepZ : d == 6 ? (G.D == 2 ? kKSweepXY : kKSweepX) : kKSweepX + d);
     int rc;
     const int form = G.prm.precision == MFC_PREC_FP64        ? kFormF64
                      : G.prm.precision == MFC_PREC_FP64_FAST ? kFormF64Fast
@@ -1278,7 +1287,11 @@ int mfc_tvd_rk_step(int t_step, double dt, double *const *q_cons_ts1, double *co
     if (int rc = fields(rhs_vf, rhs, "rhs_vf")) return rc;
     if (G.prm.time_stepper > 1)
         if (int rc = fields(q_cons_ts2, q2, "q_cons_ts(2)")) return rc;
-    if (int rc = bc_fill(q1)) return rc;
+    // each stage in one kernel, which reads its input's ghost cells through the
+    // boundary codes; it fills them only in the caller's arrays
+    const bool one = G.prm.time_stepper > 1 && stage_in_one();
+    if (!one || q_prim_vf || t_step == G.prm.t_step_stop)
+        if (int rc = bc_fill(q1)) return rc;
     if (t_step == G.prm.t_step_stop) return 1;
     if (q_prim_vf) {
         if (int rc = fields(q_prim_vf, qp, "q_prim_vf")) return rc;
@@ -1296,12 +1309,23 @@ int mfc_tvd_rk_step(int t_step, double dt, double *const *q_cons_ts1, double *co
     // a stage whose output is the next stage's input, with its ghost cells
     const bool filled = sweeps_fill_ghosts();
     auto stage = [&](const Fields &in, int rk, const Fields &out) -> int {
-        if (int rc = sweeps(in, rhs, rk, &q1, &out, dt, filled)) return rc;
-        return filled ? 0 : bc_fill(out);
+        if (one) {
+            SweepArgs a = stage_args();
+            a.qin = in;
+            a.qbase = q1;
+            a.qout = out;
+            a.dt = dt;
+            a.rk = rk;
+            a.ghosts = in.v[0] != G.scratch_state;
+            return sweep(6, a);
+        }
+        const bool next = out.v[0] != q1.v[0]; // another stage follows
+        if (int rc = sweeps(in, rhs, rk, &q1, &out, dt, filled && next)) return rc;
+        return filled || !next ? 0 : bc_fill(out);
     };
     if (G.prm.time_stepper == 2) {
         if (int rc = stage(q1, kRkEuler, q2)) return rc;
-        return sweeps(q2, rhs, kRk2Final, &q1, &q1, dt);
+        return stage(q2, kRk2Final, q1);
     }
     if (!G.scratch_state) HIPCHK(hipMalloc(&G.scratch_state, sizeof(double) * G.S * G.ng));
     Fields q3;
@@ -1311,7 +1335,7 @@ int mfc_tvd_rk_step(int t_step, double dt, double *const *q_cons_ts1, double *co
     // stencil and writes a different array, or only its own cell of q1.
     if (int rc = stage(q1, kRkEuler, q3)) return rc;
     if (int rc = stage(q3, kRk3Stage2, q2)) return rc;
-    return sweeps(q2, rhs, kRk3Stage3, &q1, &q1, dt);
+    return stage(q2, kRk3Stage3, q1);
 }
 
 int mfc_cons_to_prim(double *const *q_cons_vf, double *const *q_prim_vf) {

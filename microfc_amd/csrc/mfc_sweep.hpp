@@ -92,7 +92,7 @@ struct SweepArgs {
     int rl; // entries per row of the outer index (k_march)
     // the RK stage's ghost cells: filled with its output by the sweep that
     // writes it (the stage output is then the next stage's input), from the
-    // boundary codes of every direction
+    // boundary codes of every direction; k_stage fills its input's
     int ghosts;
     int bcs[3][2];
 };
@@ -283,6 +283,22 @@ __device__ __forceinline__ void finish_load_adv(const SweepArgs &a, Off go, Off 
 #pragma unroll
     for (int v = 0; v < S; ++v)
         if (v >= a.base_lo && v < a.base_hi) f.base[v] = el(a.qbase.v[v], go);
+}
+
+// Source index of a ghost coordinate for one direction's boundary condition
+// (m_rhs.fpp:692-905): <= -3 extrapolation, -2 reflection, -1 periodic.
+__device__ __forceinline__ int bc_source(int bcb, int bce, int s, int i, bool &flip) {
+    if (i < 0) {
+        if (bcb <= -3) return 0;
+        if (bcb == -2) { flip = !flip; return -i - 1; }
+        return s + 1 + i;
+    }
+    if (i > s) {
+        if (bce <= -3) return s;
+        if (bce == -2) { flip = !flip; return 2 * s + 1 - i; }
+        return i - (s + 1);
+    }
+    return i;
 }
 
 // Ghost cells that copy interior cell i of a direction with last index s,

@@ -7,13 +7,15 @@ smallest grids of each WENO order and on cell counts that leave partial tiles.
 Bars: the plain form is bitwise the oracle's step; the contracted form is
 within 1e-12 (helpers.state_linf); the FP32-bulk and the untrained learned form
 within 1e-3 of each variable's scale, as for their right-hand sides."""
+import copy
+
 import numpy as np
 import pytest
 
 from microfc_amd import PREC_FP32_BULK, PREC_FP32_LEARNED, PREC_FP64, PREC_FP64_FAST, RhsModule, ic, learned
 from oracle import oracle as O
 
-from helpers import perturbed, say, state_linf, to_oracle
+from helpers import perturbed, say, state_linf, stretched_grids, to_oracle
 
 pytestmark = pytest.mark.gpu
 
@@ -69,3 +71,45 @@ def test_step_with_every_boundary(gpu, m, n, order, stepper, precision):
                 assert np.all(np.isfinite(got)) and err.max() <= 1e-3
         finally:
             mod.finalize()
+
+
+@pytest.mark.parametrize("precision", [PREC_FP64, PREC_FP64_FAST])
+@pytest.mark.parametrize("m,n,stretched,fluids", [(61, 0, False, 1), (62, 0, True, 2), (31, 29, True, 2), (32, 30, False, 1),
+                                                  (47, 38, True, 1), (95, 49, False, 2)])
+def test_small_steps_in_one_kernel_per_stage(gpu, m, n, stretched, fluids, precision):
+    """The kernel that takes a whole stage of a small case, at whole tiles (62
+    cells in 1D, 16 x 10 in 2D), one cell less and one more, on equal and
+    unequal widths: the bars above."""
+    torch = gpu
+    bx, by = (-2, -4), (-4, -2)
+    prm, grids, q = _case(m, n, 5, 3, bx, by)
+    if fluids == 1:
+        prm1 = copy.deepcopy(prm)
+        prm1.num_fluids, prm1.gammas, prm1.pi_infs = 1, [2.5], [0.0]
+        D = prm.num_dims
+        prim = np.stack([1.0 + 0.3 * np.sin(7 * i + ic.mesh(prm, grids)[0]) for i in range(D + 2)] +
+                        [np.ones(prm.interior_shape[1:])])
+        prm, q = prm1, ic.ghosted(prm1, ic.prim_to_cons(prm1, prim))
+    if stretched:
+        grids = stretched_grids(prm)
+    oc = to_oracle(prm)
+    prm.precision = precision
+    mod = RhsModule(prm, grids)
+    try:
+        qd = torch.from_numpy(q.copy()).cuda()
+        q2, rd = mod.new_field(), mod.new_field(ghosted=False)
+        dt = mod.cfl_dt(qd, 0.3)
+        qo = q.copy()
+        for _ in range(2):
+            mod.s_tvd_rk(0, (qd, q2), None, rd, dt)
+            O.tvd_rk_step(oc, grids, dt, qo)
+        mod.sync()
+        got, want = prm.interior(qd.cpu().numpy()), prm.interior(qo)
+        err = state_linf(prm, got, want, q)
+        say(f"[small stage] {m + 1}x{n + 1} fluids {fluids} stretched {stretched} precision {precision} {err.max():.2e}")
+        if precision == PREC_FP64:
+            assert np.array_equal(got, want)
+        else:
+            assert err.max() <= 2e-12  # two steps
+    finally:
+        mod.finalize()
