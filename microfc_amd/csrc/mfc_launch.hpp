@@ -11,7 +11,7 @@ namespace mfc {
 
 struct SweepLaunch {
     int dir;       // 0, 1, 2; 3: the fused x and y sweep (k_sweep_xy); 4: the x and y march; 5: the z march;
-                   // 6: an RK stage in one kernel (k_stage)
+                   // 6: an RK stage in one kernel (k_stage); 7: the y march
     int num_dims;  // 1..3
     int weno_order;
     int precision; // MFC_PREC_*
@@ -29,10 +29,13 @@ int launch_sweep(const SweepLaunch &L, const SweepArgs &a, hipStream_t st);
     static int launch_nf##NF##_dwrm(int dir, const SweepArgs &a, hipStream_t st) {                      \
         const dim3 grid((unsigned)a.nblocks);                                                           \
         if (dir == 4) {                                                                                 \
-            if constexpr (NF <= kMarchMaxFluids && D >= 2 && WO == 5 && !ML && (sizeof(R) == 8 || !UNI)) hipLaunchKernelGGL((k_march<NF, D, 1, R, true, UNI>), grid, dim3(64), 0, st, a); \
+            if constexpr (NF <= kMarchMaxFluidsXY && D >= 2 && WO == 5 && !ML && (sizeof(R) == 8 || !UNI)) hipLaunchKernelGGL((k_march<NF, D, 1, R, true, UNI>), grid, dim3(64), 0, st, a); \
             else return -1;                                                                             \
         } else if (dir == 5) {                                                                          \
-            if constexpr (NF <= kMarchMaxFluids && D == 3 && WO == 5 && !ML) hipLaunchKernelGGL((k_march<NF, 3, 2, R, false, UNI>), grid, dim3(64), 0, st, a); \
+            if constexpr (NF <= kMarchMaxFluidsZ && D == 3 && WO == 5 && !ML) hipLaunchKernelGGL((k_march<NF, 3, 2, R, false, UNI>), grid, dim3(64), 0, st, a); \
+            else return -1;                                                                             \
+        } else if (dir == 7) {                                                                          \
+            if constexpr (NF > kMarchMaxFluidsXY && NF <= kMarchMaxFluidsZ && D == 3 && WO == 5 && !ML) hipLaunchKernelGGL((k_march<NF, 3, 1, R, false, UNI>), grid, dim3(64), 0, st, a); \
             else return -1;                                                                             \
         } else if (dir == 6) {                                                                          \
             if constexpr (NF <= kXyMaxFluids && D <= 2 && WO == 5 && !ML && sizeof(R) == 8) hipLaunchKernelGGL((k_stage<NF, D, UNI>), grid, dim3(stage_threads(NF, D)), 0, st, a); \

@@ -1,10 +1,11 @@
-// mfc_march.hpp -- marching sweeps of large WENO5 cases, one or two fluids.
+// mfc_march.hpp -- marching sweeps of large WENO5 cases, one to three fluids.
 //
 // A wave owns 64 neighbouring columns of cells and walks them along y or z
 // row by row, so a row is converted to primitive once, each face of the
 // marching direction is reconstructed and solved once (its lower flux is
 // kept for the next row), and no lane waits for another wave:
-//   * z march (MD = 2): every lane's cell is finished;
+//   * z march (MD = 2), and the y march alone (MD = 1, three fluids): every
+//     lane's cell is finished;
 //   * y march with the x faces of each row (WX): the lanes are consecutive
 //     entries of the rows of the outer index set end to end, each row with
 //     its three x ghost cells on either side; lanes 1 .. 62 finish their cell
@@ -25,6 +26,11 @@
 // -> 4.70 ms.  The z march then runs at the memory's rate (23 GB per launch,
 // 4.8 TB/s, as a large copy); the x and y march (30 GB, 4.1 TB/s) at 75 % VALU
 // busy, its two waves per SIMD waiting on LDS and memory for the rest.
+//
+// With three fluids the state of the x faces no longer fits beside the march's
+// (the ring takes 15 KB a wave, the z march 176 to 224 VGPRs): x keeps its
+// sweep, y and z march on their own.  180 x 130 x 90 stretched cells,
+// contracted: y 0.203 -> 0.130, z 0.183 -> 0.118 ms per launch.
 #pragma once
 
 #include "mfc_sweep.hpp"
@@ -33,7 +39,7 @@ namespace mfc {
 
 constexpr int kMarchCellsXY = 62, kMarchCellsZ = 64; // cells a wave can finish per row
 constexpr int kMarchHaloXY = 3;                      // x ghost cells per row end in the entry order
-constexpr int kMarchMaxFluids = 2;
+constexpr int kMarchMaxFluidsXY = 2, kMarchMaxFluidsZ = 3;
 
 inline namespace MFC_FORM {
 
@@ -67,11 +73,11 @@ __device__ __forceinline__ void hold(R (&v)[N]) {
 // (of the variables lo .. hi-1 in a spread stage) ...  Every lane loads, from
 // clamped cells where it has none to finish: loads under a branch were
 // spilled as they arrived.
-template <int NF, int D, bool WX, int M>
+template <int NF, int D, bool RHS, int M>
 __device__ __forceinline__ void march_load_acc(const SweepArgs &a, const SweepArgs &base, Off go, Off ro, int lo, int hi,
                                                FinishIn<Sys<NF, D>::S> &f) {
     constexpr int S = Sys<NF, D>::S;
-    if constexpr (D == 3 && (M == kModesAll) != WX) {
+    if constexpr (RHS) {
 #pragma unroll
         for (int v = 0; v < S; ++v) f.rhs[v] = el(a.rhs.v[v], ro);
     }
@@ -124,7 +130,7 @@ constexpr int march_waves() { return sizeof(R) == 4 ? 3 : 2; }
 
 template <int NF, int D, int MD, typename R, bool WX, bool UNI>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(march_waves<R>(), march_waves<R>()))) void k_march(const SweepArgs a) {
-    static_assert((MD == 1 && WX) || (MD == 2 && !WX && D == 3), "y march with the x faces, z march");
+    static_assert((MD == 1 && WX) || (!WX && D == 3), "y march with the x faces, y and z march");
     using Y = Sys<NF, D>;
     constexpr int S = Y::S;
     constexpr int PN = 2;
@@ -136,7 +142,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(march_waves<
     constexpr int HB = sizeof(R) == 8 ? 4 : 8; // rows per batch of the entries around the lanes'
     constexpr bool CANON = kFastF64 && sizeof(R) == 8 && UNI;
     // the RK base: the z march adds the first kBaseOnZFused variables
-    constexpr int BLO = WX && D == 3 ? kBaseOnZFused : 0, BHI = WX ? S : kBaseOnZFused;
+    constexpr int BLO = MD == 1 && D == 3 ? kBaseOnZFused : 0, BHI = MD == 1 ? S : kBaseOnZFused;
+    // whether rhs holds another direction's part: in 3D the sums begin in the
+    // z march, or in the plain form in the x and y march or the x sweep
+    constexpr bool RHS = D == 3 && (MD == 2 ? FM == kModesAll : WX ? FM != kModesAll : true);
     __shared__ R ring[3][S][RW];
     __shared__ R halo[WX ? S : 1][HB][4];
     // momentum and energy of the ring's rows, this lane's cell
@@ -279,7 +288,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(march_waves<
             const int jl = max(jr, r0); // (its operands are loaded in the passes before the first finish too)
             const Off go{0, own + (unsigned)jl * (unsigned)gp}, ro{0, rown + (unsigned)jl * (unsigned)rp};
             const bool finish = jr >= r0 && fin_lane;
-            march_load_acc<NF, D, WX, FM>(args(), fresh_args(), go, ro, BLO, BHI, fin);
+            march_load_acc<NF, D, RHS, FM>(args(), fresh_args(), go, ro, BLO, BHI, fin);
             if constexpr (!WX) {
                 march_load_in<NF, D, R, WX, FM>(args(), go, fin);
             }

@@ -87,6 +87,11 @@ constexpr int kMarchSlots = 8 * 256, kMarchRowsMin = 16;
 //    0.92, 4096^2 7.41 -> 5.74, 96^3 0.77 -> 0.79, 200^3 6.74 -> 4.93; FP32 bulk
 //    1024^2 0.26 -> 0.29, 2048^2 1.22 -> 0.86, 96^3 0.41 -> 0.48, 200^3 4.10 ->
 //    3.33.
+//  * three fluids, other widths, y and z against the separate sweeps:
+//    contracted 150 x 112 x 92 1.38 -> 1.12, 180 x 130 x 90 1.79 -> 1.40; plain
+//    150 x 112 x 92 1.86 -> 1.60; FP32 bulk 200^3, z alone 4.93 -> 4.81 (with y
+//    4.88); equal widths 256^3, z alone: contracted 8.70 -> 8.26 (with y 8.41),
+//    plain 14.3 -> 13.7.
 // The FP32-bulk form on equal widths keeps its tiles (300 x 250 x 200 4.75 ->
 // 4.91): with half the LDS and registers they fill the SIMDs already.
 constexpr double kMarchUniform2D = 8e6, kMarchUniform3D = 3e6, kMarchPerCell = 1.5e6;
@@ -806,11 +811,11 @@ SweepArgs xy_args() {
 }
 
 // Arguments of a march (k_march): d = 4 the y march with the x faces, d = 5
-// the z march.
+// the z march, d = 7 the y march alone.
 SweepArgs march_args(int d) {
-    SweepArgs a = d == 4 ? xy_args() : sweep_args(2);
-    const int cells = d == 4 ? kMarchCellsXY : kMarchCellsZ, rows = d == 4 ? G.prm.n + 1 : G.prm.p + 1;
-    const int other = d == 4 ? G.prm.p + 1 : G.prm.n + 1;
+    SweepArgs a = d == 4 ? xy_args() : sweep_args(d == 5 ? 2 : 1);
+    const int cells = d == 4 ? kMarchCellsXY : kMarchCellsZ, rows = d == 5 ? G.prm.p + 1 : G.prm.n + 1;
+    const int other = d == 5 ? G.prm.n + 1 : G.prm.p + 1;
     if (d == 4) {
         a.coef2 = G.dir[1].coef;
         a.ncell2 = G.dir[1].s + 2 * G.b + 1;
@@ -834,21 +839,24 @@ SweepArgs march_args(int d) {
     return a;
 }
 
-// Whether the x and y directions (d = 4) or the z direction (d = 5) of a
-// WENO5 case of the plain, contracted or FP32-bulk form run as a march.
+// Whether the x and y directions (d = 4), the z direction (d = 5) or with
+// three fluids the y direction (d = 7) of a WENO5 case of the plain,
+// contracted or FP32-bulk form run as a march.
 bool marches(int d) {
     if (G.visc || G.prm.precision == MFC_PREC_FP32_LEARNED || G.prm.weno_order != 5 ||
-        G.prm.num_fluids > kMarchMaxFluids || G.D < (d == 4 ? 2 : 3))
+        G.prm.num_fluids > (d == 4 ? kMarchMaxFluidsXY : kMarchMaxFluidsZ) ||
+        (d == 7 && G.prm.num_fluids <= kMarchMaxFluidsXY) || G.D < (d == 4 ? 2 : 3))
         return false;
     if (G.ng * (long)sizeof(double) >= (1L << 32)) return false; // 32-bit byte offsets within a variable
-    const bool uni = d == 4 ? G.dir[0].uniform && G.dir[1].uniform : G.dir[2].uniform;
-    if (uni && G.prm.precision == MFC_PREC_FP32_BULK) return false;
+    const bool uni = d == 4 ? G.dir[0].uniform && G.dir[1].uniform : G.dir[d == 5 ? 2 : 1].uniform;
+    if (uni && (d == 7 || G.prm.precision == MFC_PREC_FP32_BULK)) return false;
+    if (d == 7 && G.prm.precision == MFC_PREC_FP32_BULK) return false;
     if ((double)G.nint < (!uni ? kMarchPerCell : G.D == 2 ? kMarchUniform2D : kMarchUniform3D)) return false;
     // short rows or few of them: the lanes and rows a march adds at the ends
     // would outweigh what it saves
     const SweepArgs a = march_args(d);
     return a.chunk >= kMarchRowsMin &&
-           (double)G.nint / (d == 4 ? G.prm.n + 1 : G.prm.p + 1) >=
+           (double)G.nint / (d == 5 ? G.prm.p + 1 : G.prm.n + 1) >=
                0.85 * a.ntile * (d == 4 ? kMarchCellsXY : kMarchCellsZ);
 }
 
@@ -878,14 +886,16 @@ bool stage_in_one() {
 }
 
 // d = 0, 1, 2: one direction; d = 3: the fused x and y sweep; d = 4, 5: the
-// marches; d = 6: an RK stage in one kernel.
+// marches; d = 6: an RK stage in one kernel; d = 7: the y march.
 int sweep(int d, SweepArgs &a) {
     SweepLaunch L{d, G.D, G.prm.weno_order, G.prm.precision};
     if (G.prm.precision == MFC_PREC_FP32_LEARNED) {
         a.mlp = mlp_frags();
         if (!a.mlp) return fail(-4, "learned weights requested but mfc_mlp_init has not been called");
     }
-    TimedScope ts(d == 3 || d == 4 ? kKSweepXY : d == 5 ? kKSweepZ : d == 6 ? (G.D == 2 ? kKSweepXY : kKSweepX) : kKSweepX + d);
+    static constexpr int kinds[] = {kKSweepX, kKSweepX + 1, kKSweepX + 2, kKSweepXY, kKSweepXY, kKSweepZ, kKSweepXY,
+                                    kKSweepX + 1};
+    TimedScope ts(d == 6 && G.D == 1 ? kKSweepX : kinds[d]);
     int rc;
     const int form = G.prm.precision == MFC_PREC_FP64        ? kFormF64
                      : G.prm.precision == MFC_PREC_FP64_FAST ? kFormF64Fast
@@ -1021,7 +1031,7 @@ int sweeps(const Fields &qin, const Fields &rhs, int rk, const Fields *qbase, co
     // The contracted and FP32-bulk forms, WENO5, one or two fluids, fuse the y
     // and x sweeps on grids uniform in x and y (k_sweep_xy) or large enough for
     // a march (k_march): in 3D after the z sweep, in 2D alone.
-    const bool march = marches(4), marchz = marches(5);
+    const bool march = marches(4), marchz = marches(5), marchy = marches(7);
     const bool fuse = reverse && kFuseXY && G.D >= 2 &&
                       (G.prm.precision == MFC_PREC_FP64_FAST || G.prm.precision == MFC_PREC_FP32_BULK) &&
                       G.prm.weno_order == 5 && G.prm.num_fluids <= kXyMaxFluids &&
@@ -1089,7 +1099,8 @@ int sweeps(const Fields &qin, const Fields &rhs, int rk, const Fields *qbase, co
     }
     for (int k = 0; k < G.D; ++k) {
         const int d = reverse ? G.D - 1 - k : k;
-        SweepArgs a = sweep_args(d);
+        const int ld = d == 2 && marchz ? 5 : d == 1 && marchy ? 7 : d;
+        SweepArgs a = ld != d ? march_args(ld) : sweep_args(d);
         a.qin = qin;
         a.rhs = rhs;
         a.accumulate = k > 0;
@@ -1106,14 +1117,14 @@ int sweeps(const Fields &qin, const Fields &rhs, int rk, const Fields *qbase, co
             a.fold = k == 0 ? 1 : last ? 3 : 2;
             // cb*base: in 3D variables [0, kBaseOnZ) on the z sweep, the rest
             // on y; in 2D all on y (the first sweep)
-            const int split = G.D == 3 ? kBaseOnZ : 0;
+            const int split = G.D == 3 ? marchz || marchy ? kBaseOnZFused : kBaseOnZ : 0;
             if (cb != 0.0 && k == 0 && G.D == 3) a.base_lo = 0, a.base_hi = split;
             if (cb != 0.0 && k == G.D - 2) a.base_lo = split, a.base_hi = G.S;
             a.cb = cb;
             a.ci = ci;
             a.cdt = cdt;
         }
-        if (int rc = G.visc ? viscous(d, qin, rhs, a) : sweep(d, a)) return rc;
+        if (int rc = G.visc ? viscous(d, qin, rhs, a) : sweep(ld, a)) return rc;
     }
     return 0;
 }
