@@ -36,6 +36,9 @@ using namespace mfc;
 
 constexpr int kReduceBlocks = 8192; // the stability pass: 32 blocks of 256 threads per CU
 constexpr int kMaxDevices = 64;
+// No result of the CFL reduction: a signalling NaN, which no arithmetic returns.
+constexpr uint64_t kPending = 0x7FF4A5A5A5A5A5A5ull;
+constexpr long kPolls = 100000;
 
 // Block partials of the allocation-free CFL reduction (mfc_cfl_dt_noalloc):
 // one copy of this array per GPU, 64 KiB, held until the process ends.  In
@@ -487,7 +490,7 @@ template <int T> __device__ __forceinline__ double block_max(double mx) {
 // result is pinned host memory.  With the partials reduced by a kernel of
 // their own and the value copied to pageable memory, the call took 34 instead
 // of 24 us (200^2 cells), 38 instead of 30 us (768^2), 210 instead of 197 us
-// (4096^2).
+// (4096^2); then the host stopped waiting for the stream (icfl_reduce).
 constexpr int kCflThreads = 512, kCflChunk = 2 * kCflThreads, kCflBlocks = 512;
 template <int NF, int D, bool FROM_CONS>
 __global__ __launch_bounds__(kCflThreads) void k_icfl(Fields q, Eos eos, Box x, const double *dx, const double *dy,
@@ -540,7 +543,7 @@ __global__ __launch_bounds__(kCflThreads) void k_icfl(Fields q, Eos eos, Box x, 
     for (unsigned t = threadIdx.x; t < gridDim.x; t += kCflThreads)
         mx = max_nan(mx, __hip_atomic_load(&partials[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
     mx = block_max<kCflThreads>(mx);
-    if (threadIdx.x == 0) *result = mx;
+    if (threadIdx.x == 0) __hip_atomic_store(result, mx, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Stability criteria of one cell (m_data_output.fpp:214-263) from its
@@ -1373,8 +1376,11 @@ static int icfl_reduce(double *const *q, bool from_cons, double dt, double *out,
     const int nb = (int)std::min<long>(kCflBlocks, (G.nint + kCflChunk - 1) / kCflChunk);
     if (!partials || nb > capacity)
         return fail(-1, "CFL reduction needs %d partials, the buffer holds %d", nb, capacity);
+    *(volatile uint64_t *)G.result = kPending;
+    int rc;
+    {
     TimedScope ts(timed ? kKIcfl : -1);
-    const int rc = dispatch_nf_d([&](auto NF, auto D) -> int {
+    rc = dispatch_nf_d([&](auto NF, auto D) -> int {
         if (from_cons)
             hipLaunchKernelGGL((k_icfl<decltype(NF)::value, decltype(D)::value, true>), dim3(nb), dim3(kCflThreads), 0,
                                G.stream, f, e, x, dxs[0], dxs[1], dxs[2], dt, G.nint, partials, G.count, G.result);
@@ -1384,8 +1390,16 @@ static int icfl_reduce(double *const *q, bool from_cons, double dt, double *out,
         HIPCHK(hipGetLastError());
         return 0;
     });
+    }
     if (rc) return rc;
-    HIPCHK(hipStreamSynchronize(G.stream));
+    // The kernel's one store to it, seen as it arrives: the stream's
+    // synchronisation returned 5 us later (the call on 200^2 cells 23.6 ->
+    // 18.2 us).  The kernels before it on the stream have then ended.  After
+    // kPolls looks, a millisecond or two, the call waits for the stream, which
+    // also reports errors.
+    volatile uint64_t *r = (volatile uint64_t *)G.result;
+    for (long n = 0; n < kPolls && *r == kPending; ++n) __builtin_ia32_pause();
+    if (*r == kPending) HIPCHK(hipStreamSynchronize(G.stream));
     *out = *(volatile double *)G.result;
     return 0;
 }
