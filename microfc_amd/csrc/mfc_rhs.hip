@@ -485,13 +485,20 @@ template <int T> __device__ __forceinline__ double block_max(double mx) {
 // last reduces the partials (count wraps to 0 with it, ready for the next
 // call).  A block takes chunks of kCflChunk consecutive interior cells (x
 // fastest), two per thread with both cells' loads issued before either is
-// converted.  At most two blocks per compute unit: the counter takes 10 ns a
-// block (768^2 cells: 1152 blocks of 256 threads took 37 us with the call).
+// converted.  Two blocks per compute unit on small grids, since the counter
+// takes 10 ns a block (the call with 768^2 cells in 1152 blocks of 256 threads
+// took 37 us, in 512 of 512 30 us; 1500^2 cells 48.7 us in 2048 blocks, 38.3
+// in 512), and up to eight on large ones, where a block takes eight chunks and
+// more (320^3 cells 407 us in 512 blocks, 391 in 2048).
 // result is pinned host memory.  With the partials reduced by a kernel of
 // their own and the value copied to pageable memory, the call took 34 instead
 // of 24 us (200^2 cells), 38 instead of 30 us (768^2), 210 instead of 197 us
 // (4096^2); then the host stopped waiting for the stream (icfl_reduce).
-constexpr int kCflThreads = 512, kCflChunk = 2 * kCflThreads, kCflBlocks = 512;
+constexpr int kCflThreads = 512, kCflChunk = 2 * kCflThreads, kCflBlocks = 2048;
+// Blocks for so many chunks.
+int cfl_blocks(long chunks) {
+    return (int)std::min<long>(kCflBlocks, std::max(std::min(chunks, 512L), chunks / 8));
+}
 template <int NF, int D, bool FROM_CONS>
 __global__ __launch_bounds__(kCflThreads) void k_icfl(Fields q, Eos eos, Box x, const double *dx, const double *dy,
                                               const double *dz, double dt, long nint, double *partials,
@@ -1373,7 +1380,7 @@ static int icfl_reduce(double *const *q, bool from_cons, double dt, double *out,
     const Box x = box();
     const Eos e = eos();
     double *dxs[3] = {G.dir[0].ds_dev, G.dir[1].ds_dev, G.dir[2].ds_dev};
-    const int nb = (int)std::min<long>(kCflBlocks, (G.nint + kCflChunk - 1) / kCflChunk);
+    const int nb = cfl_blocks((G.nint + kCflChunk - 1) / kCflChunk);
     if (!partials || nb > capacity)
         return fail(-1, "CFL reduction needs %d partials, the buffer holds %d", nb, capacity);
     *(volatile uint64_t *)G.result = kPending;
