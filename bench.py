@@ -38,19 +38,18 @@ FP64_PEAK_TFLOPS = 78.6
 # and its VALU-busy fraction (SQ_ACTIVE_INST_VALU * 4 / (1024 CU-SIMDs *
 # GRBM_GUI_ACTIVE / 8)), with the profile summary they come from.  Other
 # workloads report null.
-_P512 = "profiles/sweep_kernels_shock_droplet_3d_512_fp64_fast.md"
+_P512 = "profiles/march_kernels_shock_droplet_3d_512_fp64_fast.md"
 _P2048 = "profiles/sweep_kernels_shock_bubble_2d_2048_fp64_fast.md"
 PROFILED = {
     ("shock_droplet_3d", 512, "fp64_fast", "sweep_xy"): {
-        "traffic": 18.89e9 + 8.60e9, "valu_busy": 0.80,
-        "limiter": "VALU issue (FP64), not HBM (27.5 GB at 3.1 TB/s)", "profile": _P512},
+        "traffic": 21.77e9 + 8.98e9, "valu_busy": 0.75,
+        "limiter": "VALU issue (FP64) and memory: 30.8 GB at 4.2 TB/s, two waves per SIMD", "profile": _P512},
     ("shock_droplet_3d", 512, "fp64_fast", "sweep_z"): {
-        "traffic": 13.86e9 + 8.59e9, "valu_busy": 0.69,
-        "limiter": "VALU issue in RK stage 1 (80 % busy); with 6 RK-base variables in stages 2 and 3, 24.8 GB at "
-                   "4.2 TB/s", "profile": _P512},
+        "traffic": 15.16e9 + 8.59e9, "valu_busy": 0.55,
+        "limiter": "HBM: 23.8 GB at 4.9 TB/s, the rate of a large copy", "profile": _P512},
     ("shock_bubble_2d", 2048, "fp64_fast", "sweep_xy"): {
-        "traffic": 453.1e6 + 236.0e6, "valu_busy": 0.67,
-        "limiter": "VALU issue and latency (63-74 % busy, four waves per SIMD), not HBM", "profile": _P2048},
+        "traffic": 393.5e6 + 236.7e6, "valu_busy": 0.64,
+        "limiter": "VALU issue and latency (63-67 % busy, four waves per SIMD), not HBM", "profile": _P2048},
 }
 
 DEFAULT_PRECISION = "fp64_fast"
@@ -83,13 +82,11 @@ def sweep_bytes_per_step(prm, fused=False):
     or, in the contracted FP64, FP32-bulk and learned forms of a 2D/3D case,
     which spread the stage over the sweeps, by the y sweep (in 3D its first
     BASE_ON_Z variables by the z sweep).  Viscous runs use the
-    viscous kernels in place of the sweeps: per direction the face kernel
-    reads the stencil input and writes a face record (HLLC flux, contact
-    velocity, viscous flux: S+2+D doubles), the finish reads it and the
-    volume fractions, and reads/writes rhs like a sweep (or, in the last
-    direction, reads the RK base and stage input and writes the output).
-    With weno_Re_flux the velocity-gradient planes and their face averages
-    add their passes.  fused: the fused x and y sweep (sweep_xy) reads the
+    viscous kernels in place of the sweeps: per direction one kernel reads
+    the stencil input and reads/writes rhs like a sweep (or, in the last
+    direction, reads the RK base and writes the output).  With weno_Re_flux
+    the pass that writes the velocity-gradient planes comes first, and each
+    direction reads them.  fused: the fused x and y sweep (sweep_xy) reads the
     stencil input once; in the contracted and FP32-bulk forms it comes after
     the z sweep in 3D, reads the z sweep's rhs and its part of the RK base
     and writes the stage output; in the plain form it comes first, writing
@@ -103,13 +100,11 @@ def sweep_bytes_per_step(prm, fused=False):
         total = 0
         for d in range(D):
             first, last = d == 0, d == D - 1
-            per = S + 2 * (S + 2 + D) + NF + (0 if first else S) + (3 * S if last else S)
+            per = S + (0 if first else S) + (2 * S if last else S)
             if prm.weno_Re_flux:
-                # the gradient pass of direction d reads the densities and
-                # momenta and writes D gradient planes; the face-average pass
-                # reads the D*D planes and writes D*D face values, which the
-                # face kernel reads
-                per += (NF + 2 * D) + 3 * D * D
+                # the gradient pass reads the densities and momenta and
+                # writes the D*D planes, once; each direction reads them
+                per += (NF + D + D * D if first else 0) + D * D
             total += 3 * 8 * per
         out["viscous"] = total
         return out
@@ -312,7 +307,7 @@ def main():
                      "profile": prof.get("profile")},
         # the step's compulsory state traffic, and the bytes this design's
         # kernels must move (the sweep_bytes_per_step model: rhs partials, RK
-        # base, and in viscous runs the face records and finish passes)
+        # base, and in viscous runs the velocity-gradient planes)
         "step_hbm": {"algorithmic_bytes_per_cell_step": 64 * S, "achieved_GBps": step_bytes * args.steps / sec / 1e9,
                      "frac": step_bytes * args.steps / sec / 1e9 / HBM_PEAK_GBS,
                      "design_bytes_per_cell_step": sum(per_step.values()),

@@ -25,6 +25,9 @@
 //    wave hold one column, thread (x, c) reconstructs both faces of cell c,
 //    the neighbouring face value moves one lane within the column, and the
 //    fluxes go through LDS to the x-fastest layout (K - 2 cells per column).
+//  * k_sweep_xy (x and y together on grids uniform in both).
+// Large cases march instead (mfc_march.hpp), and small 1D and 2D ones take an
+// RK stage in one kernel (mfc_stage.hpp).
 #pragma once
 
 #include "mfc_device.hpp"
