@@ -4,6 +4,7 @@
 #pragma once
 
 #include "mfc_march.hpp"
+#include "mfc_rows.hpp"
 #include "mfc_stage.hpp"
 #include "mfc_sweep.hpp"
 
@@ -11,7 +12,8 @@ namespace mfc {
 
 struct SweepLaunch {
     int dir;       // 0, 1, 2; 3: the fused x and y sweep (k_sweep_xy); 4: the x and y march; 5: the z march;
-                   // 6: an RK stage in one kernel (k_stage); 7: the y march
+                   // 6: an RK stage in one kernel (k_stage); 7: the y march;
+                   // 8: the x sweep along rows (k_rows_x)
     int num_dims;  // 1..3
     int weno_order;
     int precision; // MFC_PREC_*
@@ -33,6 +35,9 @@ int launch_sweep(const SweepLaunch &L, const SweepArgs &a, hipStream_t st);
             else return -1;                                                                             \
         } else if (dir == 5) {                                                                          \
             if constexpr (NF <= kMarchMaxFluidsZ && D == 3 && WO == 5 && !ML) hipLaunchKernelGGL((k_march<NF, 3, 2, R, false, UNI>), grid, dim3(64), 0, st, a); \
+            else return -1;                                                                             \
+        } else if (dir == 8) {                                                                          \
+            if constexpr (NF <= kRowsMaxFluids && D >= 2 && WO == 5 && !ML && !UNI && sizeof(R) == 8) hipLaunchKernelGGL((k_rows_x<NF, D>), grid, dim3(64), 0, st, a); \
             else return -1;                                                                             \
         } else if (dir == 7) {                                                                          \
             if constexpr (NF > kMarchMaxFluidsXY && NF <= kMarchMaxFluidsZ && D == 3 && WO == 5 && !ML) hipLaunchKernelGGL((k_march<NF, 3, 1, R, false, UNI>), grid, dim3(64), 0, st, a); \

@@ -870,6 +870,40 @@ bool marches(int d) {
                0.85 * a.ntile * (d == 4 ? kMarchCellsXY : kMarchCellsZ);
 }
 
+// Arguments of k_rows_x.
+SweepArgs rows_args() {
+    SweepArgs a = sweep_args(0);
+    a.rl = G.prm.m + 7;
+    a.ntile = (int)(((long)a.rl * (G.prm.p + 1) + kRowsCells - 4) / kRowsCells);
+    // chunks as in march_args; a chunk costs about a row more than it finishes
+    // (the coefficients' loads)
+    const int rows = G.prm.n + 1;
+    double best = 0.0;
+    for (int L = 1; L <= std::min(rows, 32); ++L) {
+        const int nc = (rows + L - 1) / L;
+        const double cost = std::max(1.0, (double)a.ntile * nc / kMarchSlots + 0.5) * (L + 1);
+        if (best == 0.0 || cost < best) best = cost, a.chunk = L, a.nchunk = nc;
+    }
+    a.nblocks = (long)a.ntile * a.nchunk;
+    return a;
+}
+
+// Whether the x direction of a case on unequal widths runs along rows
+// (k_rows_x): from two rounds of waves with a row each.  RK3 step, plain or
+// contracted (c), x sweep -> rows: 400 x 300 cells (2400 sets of columns and
+// rows) 106 -> 104 us, 600 x 500 (5500) 185 -> 180, 700 x 700 269 -> 247, 1000 x
+// 900 428 -> 397, c 800 x 800 219 -> 211; 70 x 60 x 60 (4800) 340 -> 287, 96^3
+// 804 -> 750, but c 60 x 56 x 50 (3300) 155 -> 156; three fluids c 60 x 50 x 40
+// 156 -> 162, 180 x 130 x 90 1436 -> 1284, plain 2080 -> 1990.
+constexpr long kRowsMin = 2 * kMarchSlots;
+bool rows_x() {
+    if (G.D < 2 || G.visc || G.prm.weno_order != 5 || G.prm.num_fluids > kRowsMaxFluids || G.dir[0].uniform ||
+        (G.prm.precision != MFC_PREC_FP64 && G.prm.precision != MFC_PREC_FP64_FAST))
+        return false;
+    if (G.ng * (long)sizeof(double) >= (1L << 32)) return false; // 32-bit byte offsets within a variable
+    return (long)rows_args().ntile * (G.prm.n + 1) >= kRowsMin;
+}
+
 // Arguments of k_stage.
 SweepArgs stage_args() {
     SweepArgs a = G.D == 2 ? xy_args() : sweep_args(0);
@@ -904,7 +938,7 @@ int sweep(int d, SweepArgs &a) {
         if (!a.mlp) return fail(-4, "learned weights requested but mfc_mlp_init has not been called");
     }
     static constexpr int kinds[] = {kKSweepX, kKSweepX + 1, kKSweepX + 2, kKSweepXY, kKSweepXY, kKSweepZ, kKSweepXY,
-                                    kKSweepX + 1};
+                                    kKSweepX + 1, kKSweepX};
     TimedScope ts(d == 6 && G.D == 1 ? kKSweepX : kinds[d]);
     int rc;
     const int form = G.prm.precision == MFC_PREC_FP64        ? kFormF64
@@ -1109,8 +1143,8 @@ int sweeps(const Fields &qin, const Fields &rhs, int rk, const Fields *qbase, co
     }
     for (int k = 0; k < G.D; ++k) {
         const int d = reverse ? G.D - 1 - k : k;
-        const int ld = d == 2 && marchz ? 5 : d == 1 && marchy ? 7 : d;
-        SweepArgs a = ld != d ? march_args(ld) : sweep_args(d);
+        const int ld = d == 2 && marchz ? 5 : d == 1 && marchy ? 7 : d == 0 && rows_x() ? 8 : d;
+        SweepArgs a = ld == d ? sweep_args(d) : ld == 8 ? rows_args() : march_args(ld);
         a.qin = qin;
         a.rhs = rhs;
         a.accumulate = k > 0;

@@ -26,7 +26,8 @@
 //    the neighbouring face value moves one lane within the column, and the
 //    fluxes go through LDS to the x-fastest layout (K - 2 cells per column).
 //  * k_sweep_xy (x and y together on grids uniform in both).
-// Large cases march instead (mfc_march.hpp), and small 1D and 2D ones take an
+// Large cases march instead (mfc_march.hpp), the x direction on unequal widths
+// goes along rows (mfc_rows.hpp), and small 1D and 2D ones take an
 // RK stage in one kernel (mfc_stage.hpp).
 #pragma once
 
