@@ -31,6 +31,11 @@ int launch_sweep(const SweepLaunch &L, const SweepArgs &a, hipStream_t st);
     static int launch_nf##NF##_dwrm(int dir, const SweepArgs &a, hipStream_t st) {                      \
         const dim3 grid((unsigned)a.nblocks);                                                           \
         if (dir == 4) {                                                                                 \
+            if constexpr (NF <= kMarchMaxFluidsXY && D >= 2 && WO == 5 && !ML && sizeof(R) == 8 && !kFastF64) \
+                if (a.prim.v[0]) {                                                                      \
+                    hipLaunchKernelGGL((k_march<NF, D, 1, R, true, UNI, true>), grid, dim3(64), 0, st, a); \
+                    return hipGetLastError() == hipSuccess ? 0 : -2;                                    \
+                }                                                                                       \
             if constexpr (NF <= kMarchMaxFluidsXY && D >= 2 && WO == 5 && !ML && (sizeof(R) == 8 || !UNI)) hipLaunchKernelGGL((k_march<NF, D, 1, R, true, UNI>), grid, dim3(64), 0, st, a); \
             else return -1;                                                                             \
         } else if (dir == 5) {                                                                          \

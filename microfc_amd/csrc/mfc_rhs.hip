@@ -365,37 +365,48 @@ __device__ __forceinline__ long box_off(const Box &x, int i, int j, int k) {
 // round trip waits for the one before), and the cell's indices come from
 // 32-bit divisions.  200 x 150 cells, 7 variables 4.7 -> 3.7 us, 1000 cells 3.3 -> 2.8 us.
 constexpr int kBcVars = 8; // variables per round trip
-__global__ __launch_bounds__(256) void k_bc_fill(Fields q, int S, int momxb, Box x, int bxb, int bxe, int byb, int bye,
-                                                 int bzb, int bze, unsigned n0, unsigned n1, unsigned n2) {
-    const int slab = blockIdx.y;
-    const unsigned t = blockIdx.x * 256u + threadIdx.x;
+struct BcCodes {
+    int xb, xe, yb, ye, zb, ze;
+};
+// Ghost cell t of slab `slab`: its offset, its source's and the mirrored
+// directions; false past the slab's end.
+__device__ __forceinline__ bool bc_cell(const Box &x, const BcCodes &bc, int slab, unsigned t, unsigned n0, unsigned n1,
+                                        unsigned n2, long &dst, long &src, bool &fx, bool &fy, bool &fz) {
     int i, j, k;
     const unsigned gx = 2 * x.b, gy = 2 * x.bj;
     const unsigned NY = x.n + 1 + gy, NX = x.m + 1;
     if (slab == 0) {
-        if (t >= n0) return;
+        if (t >= n0) return false;
         const unsigned r = t / gx, gi = t - r * gx, kk = r / NY, jj = r - kk * NY;
         i = (int)gi < x.b ? (int)gi - x.b : x.m + 1 + ((int)gi - x.b);
         j = (int)jj - x.bj;
         k = (int)kk - x.bk;
     } else if (slab == 1) {
-        if (t >= n1) return;
+        if (t >= n1) return false;
         const unsigned r = t / NX, ii = t - r * NX, kk = r / gy, gj = r - kk * gy;
         i = (int)ii;
         j = (int)gj < x.bj ? (int)gj - x.bj : x.n + 1 + ((int)gj - x.bj);
         k = (int)kk - x.bk;
     } else {
-        if (t >= n2) return;
+        if (t >= n2) return false;
         const unsigned r = t / NX, ii = t - r * NX, NI = x.n + 1, gk = r / NI, jj = r - gk * NI;
         i = (int)ii;
         j = (int)jj;
         k = (int)gk < x.bk ? (int)gk - x.bk : x.p + 1 + ((int)gk - x.bk);
     }
-    bool fx = false, fy = false, fz = false;
-    const int si = bc_source(bxb, bxe, x.m, i, fx);
-    const int sj = x.bj ? bc_source(byb, bye, x.n, j, fy) : j;
-    const int sk = x.bk ? bc_source(bzb, bze, x.p, k, fz) : k;
-    const long dst = box_off(x, i, j, k), src = box_off(x, si, sj, sk);
+    fx = fy = fz = false;
+    const int si = bc_source(bc.xb, bc.xe, x.m, i, fx);
+    const int sj = x.bj ? bc_source(bc.yb, bc.ye, x.n, j, fy) : j;
+    const int sk = x.bk ? bc_source(bc.zb, bc.ze, x.p, k, fz) : k;
+    dst = box_off(x, i, j, k);
+    src = box_off(x, si, sj, sk);
+    return true;
+}
+__global__ __launch_bounds__(256) void k_bc_fill(Fields q, int S, int momxb, Box x, BcCodes bc, unsigned n0, unsigned n1,
+                                                 unsigned n2) {
+    long dst, src;
+    bool fx, fy, fz;
+    if (!bc_cell(x, bc, blockIdx.y, blockIdx.x * 256u + threadIdx.x, n0, n1, n2, dst, src, fx, fy, fz)) return;
     for (int v0 = 0; v0 < S; v0 += kBcVars) {
         double val[kBcVars];
 #pragma unroll
@@ -408,6 +419,29 @@ __global__ __launch_bounds__(256) void k_bc_fill(Fields q, int S, int momxb, Box
             const bool neg = (fx && v == momxb) || (fy && v == momxb + 1) || (fz && v == momxb + 2);
             q.v[v][dst] = neg ? -val[u] : val[u];
         }
+    }
+}
+
+// The ghost fill and the ghost cells' primitive values.
+template <int NF, int D>
+__global__ __launch_bounds__(256) void k_bc_prim(Fields q, Fields qp, Eos eos, Box x, BcCodes bc, unsigned n0,
+                                                 unsigned n1, unsigned n2) {
+    using Y = Sys<NF, D>;
+    constexpr int S = Y::S;
+    long dst, src;
+    bool f[3];
+    if (!bc_cell(x, bc, blockIdx.y, blockIdx.x * 256u + threadIdx.x, n0, n1, n2, dst, src, f[0], f[1], f[2])) return;
+    double c[S], p[S];
+#pragma unroll
+    for (int v = 0; v < S; ++v) c[v] = q.v[v][src];
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+        if (f[d]) c[Y::MOM + d] = -c[Y::MOM + d];
+    cons_to_prim<NF, D>(c, p, eos);
+#pragma unroll
+    for (int v = 0; v < S; ++v) {
+        q.v[v][dst] = c[v];
+        qp.v[v][dst] = p[v];
     }
 }
 
@@ -720,7 +754,8 @@ int dispatch_nf_d(F &&f) {
     return fail(-1, "no kernels for num_fluids=%d, num_dims=%d", nf, D);
 }
 
-int bc_fill(const Fields &q) {
+// prim: also the ghost cells' primitive values.
+int bc_fill(const Fields &q, const Fields *prim = nullptr) {
     const Box x = box();
     const long n0 = (long)(2 * x.b) * (x.n + 1 + 2 * x.bj) * (x.p + 1 + 2 * x.bk);
     const long n1 = (long)(x.m + 1) * (2 * x.bj) * (x.p + 1 + 2 * x.bk);
@@ -728,9 +763,16 @@ int bc_fill(const Fields &q) {
     const long nmax = std::max(n0, std::max(n1, n2));
     const dim3 grid((unsigned)((nmax + 255) / 256), 1 + (G.D >= 2) + (G.D >= 3)), block(256);
     TimedScope ts(kKBcFill);
-    hipLaunchKernelGGL(k_bc_fill, grid, block, 0, G.stream, q, G.S, G.prm.num_fluids, x, G.prm.bc_x_beg,
-                       G.prm.bc_x_end, G.prm.bc_y_beg, G.prm.bc_y_end, G.prm.bc_z_beg, G.prm.bc_z_end, (unsigned)n0,
-                       (unsigned)n1, (unsigned)n2);
+    const BcCodes bc{G.prm.bc_x_beg, G.prm.bc_x_end, G.prm.bc_y_beg, G.prm.bc_y_end, G.prm.bc_z_beg, G.prm.bc_z_end};
+    if (prim)
+        return dispatch_nf_d([&](auto NF, auto D) -> int {
+            hipLaunchKernelGGL((k_bc_prim<decltype(NF)::value, decltype(D)::value>), grid, block, 0, G.stream, q, *prim,
+                               eos(), x, bc, (unsigned)n0, (unsigned)n1, (unsigned)n2);
+            HIPCHK(hipGetLastError());
+            return 0;
+        });
+    hipLaunchKernelGGL(k_bc_fill, grid, block, 0, G.stream, q, G.S, G.prm.num_fluids, x, bc, (unsigned)n0, (unsigned)n1,
+                       (unsigned)n2);
     HIPCHK(hipGetLastError());
     return 0;
 }
@@ -1011,14 +1053,19 @@ bool sweeps_fill_ghosts() {
            G.prm.num_fluids <= kXyMaxFluids && G.dir[0].uniform && G.dir[1].uniform && !marches(4);
 }
 
+// Whether the x and y march can store the primitive field of its input.
+bool march_stores_prim() { return G.prm.precision == MFC_PREC_FP64 && kFuseXY && marches(4); }
+
 // All directional sweeps of one RHS evaluation on the ghost-filled field qin.
 // The last sweep either writes rhs (rk = kRkNone) or applies the RK stage.
 // Viscous runs use the viscous kernels for each direction instead, with the
 // same finish semantics.
 // ghosts: the last sweep also fills the ghost cells of *qout (the caller's
 // next stage input; sweeps_fill_ghosts).
+// prim: the x and y march also stores the interior's primitive values
+// (march_stores_prim).
 int sweeps(const Fields &qin, const Fields &rhs, int rk, const Fields *qbase, const Fields *qout, double dt,
-           bool ghosts = false) {
+           bool ghosts = false, const Fields *prim = nullptr) {
     // The plain form adds the directions in the reference's order x, y, z
     // (m_rhs.fpp:469-656; it fixes the rounding).  The contracted FP64,
     // FP32-bulk and learned forms run them in the reverse order: the sum is
@@ -1132,6 +1179,7 @@ int sweeps(const Fields &qin, const Fields &rhs, int rk, const Fields *qbase, co
         SweepArgs a = march ? march_args(4) : xy_args();
         finish(a, G.D == 2);
         a.accumulate = 0;
+        if (prim) a.prim = *prim;
         if (int rc = sweep(march ? 4 : 3, a)) return rc;
         if (G.D == 3) {
             SweepArgs z = marchz ? march_args(5) : sweep_args(2);
@@ -1324,13 +1372,17 @@ int mfc_compute_rhs(double *const *q_cons_vf, double *const *q_prim_vf, double *
     if (int rc = require_ready()) return rc;
     Fields qc, qp, rhs;
     if (int rc = fields(q_cons_vf, qc, "q_cons_vf")) return rc;
-    if (int rc = bc_fill(qc)) return rc;
+    // the primitive field from the march that converts the cells anyway
+    const bool fused = q_prim_vf && t_step != G.prm.t_step_stop && march_stores_prim();
+    if (!fused)
+        if (int rc = bc_fill(qc)) return rc;
     if (t_step == G.prm.t_step_stop) return 1;
     if (int rc = fields(rhs_vf, rhs, "rhs_vf")) return rc;
     if (q_prim_vf) {
         if (int rc = fields(q_prim_vf, qp, "q_prim_vf")) return rc;
-        if (int rc = cons_to_prim_launch(qc, qp)) return rc;
+        if (int rc = fused ? bc_fill(qc, &qp) : cons_to_prim_launch(qc, qp)) return rc;
     }
+    if (fused) return sweeps(qc, rhs, kRkNone, nullptr, nullptr, 0.0, false, &qp);
     return sweeps(qc, rhs, kRkNone, nullptr, nullptr, 0.0);
 }
 

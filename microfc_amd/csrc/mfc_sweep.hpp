@@ -99,6 +99,7 @@ struct SweepArgs {
     // boundary codes of every direction; k_stage fills its input's
     int ghosts;
     int bcs[3][2];
+    Fields prim; // k_march with PO: the primitive field of the stage input
 };
 
 // RK-base variables the z sweep adds before the fused x and y sweep
