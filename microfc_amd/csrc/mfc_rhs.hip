@@ -1262,7 +1262,8 @@ int mfc_rhs_init(const mfc_params *prm) {
     G.stream = G.own;
     HIPCHK(hipMalloc(&G.partials, sizeof(double) * 2 * kReduceBlocks));
     HIPCHK(hipMalloc(&G.count, sizeof(unsigned)));
-    HIPCHK(hipMemset(G.count, 0, sizeof(unsigned)));
+    const unsigned none = 0;
+    HIPCHK(hipMemcpy(G.count, &none, sizeof none, hipMemcpyHostToDevice));
     HIPCHK(hipHostMalloc(&G.result, sizeof(double), hipHostMallocDefault));
     {
         int dev = 0;

@@ -15,7 +15,7 @@ import pytest
 from microfc_amd import PREC_FP32_BULK, PREC_FP32_LEARNED, PREC_FP64, PREC_FP64_FAST, RhsModule, ic, learned
 from oracle import oracle as O
 
-from helpers import perturbed, say, state_linf, stretched_grids, to_oracle
+from helpers import multi_fluid_2d, perturbed, say, state_linf, stretched_grids, to_oracle
 
 pytestmark = pytest.mark.gpu
 
@@ -113,3 +113,42 @@ def test_small_steps_in_one_kernel_per_stage(gpu, m, n, stretched, fluids, preci
             assert err.max() <= 2e-12  # two steps
     finally:
         mod.finalize()
+
+
+@pytest.mark.parametrize("precision", [PREC_FP64, PREC_FP64_FAST])
+@pytest.mark.parametrize("fluids", [1, 3, 4, 5, 7, 10])
+def test_one_dimension_with_many_fluids(gpu, fluids, precision):
+    """1D steps whose sweep fills the ghost cells (three fluids and more, and
+    WENO3 with any number): the bars above."""
+    torch = gpu
+    for order, (bx0, bx1) in ((5, (-2, -4)), (5, (-1, -1)), (3, (-3, -2))):
+        prm = multi_fluid_2d(fluids, N=32)[0]
+        prm.m, prm.n, prm.weno_order = 131, 0, order
+        prm.bc_beg, prm.bc_end = (bx0, -3, -3), (bx1, -3, -3)
+        grids = ic.uniform_grids(prm)
+        X = ic.mesh(prm, grids)[0]
+        w = [1.0 + 0.5 * np.sin((5 + 2 * i) * X + i) for i in range(fluids)]
+        al = [x / sum(w) for x in w]
+        prim = np.stack([(1.0 + 0.7 * i) * al[i] for i in range(fluids)] +
+                        [10 * np.sin(6 * X + 0.2), 1e5 * (1 + 0.3 * np.cos(9 * X))] + al)
+        q = perturbed(prm, ic.ghosted(prm, ic.prim_to_cons(prm, prim)))
+        oc = to_oracle(prm)
+        prm.precision = precision
+        mod = RhsModule(prm, grids)
+        try:
+            qd = torch.from_numpy(q.copy()).cuda()
+            q2, rd = mod.new_field(), mod.new_field(ghosted=False)
+            dt = mod.cfl_dt(qd, 0.3)
+            mod.s_tvd_rk(0, (qd, q2), None, rd, dt)
+            mod.sync()
+            qo = q.copy()
+            O.tvd_rk_step(oc, grids, dt, qo)
+            got, want = prm.interior(qd.cpu().numpy()), prm.interior(qo)
+            err = state_linf(prm, got, want, q)
+            say(f"[1D ghosts] fluids {fluids} order {order} bc {bx0} {bx1} precision {precision} {err.max():.2e}")
+            if precision == PREC_FP64:
+                assert np.array_equal(got, want)
+            else:
+                assert err.max() <= 1e-12
+        finally:
+            mod.finalize()
