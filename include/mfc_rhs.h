@@ -150,9 +150,10 @@ int mfc_cfl_dt(double *const *q_cons_vf, double cfl, double *dt_out);
  * mfc_cfl_dt, bit for bit; the block partials live in a fixed 64 KiB device
  * array (8192 doubles, one copy per GPU, kept until the process ends) in
  * place of the buffer mfc_rhs_init allocates.  The reduction is a
- * grid-stride pass over at most 8192 blocks, so every grid size fits.  Calls
- * that overlap on one GPU (several host threads, or several streams set with
- * mfc_set_stream) share that array and race.  Needs mfc_rhs_init and
+ * grid-stride pass over at most 2048 blocks, so every grid size fits.  Calls
+ * of mfc_cfl_dt, mfc_cfl_dt_noalloc, mfc_icfl_max and mfc_stability_criteria
+ * from several host threads take turns: each holds the reduction's buffers
+ * until its value is on the host.  Needs mfc_rhs_init and
  * mfc_rhs_set_grid first, like mfc_cfl_dt; blocks until dt is on the host. */
 int mfc_cfl_dt_noalloc(double *const *q_cons_vf, double cfl, double *dt_out);
 

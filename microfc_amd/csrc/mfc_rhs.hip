@@ -8,6 +8,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -47,6 +48,11 @@ constexpr long kPolls = 100000;
 static __device__ __align__(256) double scratch[kReduceBlocks];
 
 namespace {
+
+// Held by the entry points that reduce over the cells, each until its value is
+// on the host: a case has one block counter and one result word (k_icfl), and
+// one array of partials for all but mfc_cfl_dt_noalloc.
+std::mutex g_reduce;
 
 // Device address of `scratch` on each GPU, looked up once per device by
 // mfc_rhs_init with that device current.
@@ -1457,7 +1463,7 @@ int mfc_cons_to_prim(double *const *q_cons_vf, double *const *q_prim_vf) {
 // The ICFL max-reduction into `partials` (capacity doubles), a grid-stride
 // pass of at most kCflBlocks blocks, so every grid size fits.  `timed`
 // records HIP events around the pass (event creation may allocate, so the
-// allocation-free entry point passes false).
+// allocation-free entry point passes false).  The caller holds g_reduce.
 static int icfl_reduce(double *const *q, bool from_cons, double dt, double *out, double *partials, int capacity,
                        bool timed) {
     if (int rc = require_ready()) return rc;
@@ -1470,6 +1476,7 @@ static int icfl_reduce(double *const *q, bool from_cons, double dt, double *out,
     const int nb = cfl_blocks((G.nint + kCflChunk - 1) / kCflChunk);
     if (!partials || nb > capacity)
         return fail(-1, "CFL reduction needs %d partials, the buffer holds %d", nb, capacity);
+    const hipStream_t st = G.stream;
     *(volatile uint64_t *)G.result = kPending;
     int rc;
     {
@@ -1477,10 +1484,10 @@ static int icfl_reduce(double *const *q, bool from_cons, double dt, double *out,
     rc = dispatch_nf_d([&](auto NF, auto D) -> int {
         if (from_cons)
             hipLaunchKernelGGL((k_icfl<decltype(NF)::value, decltype(D)::value, true>), dim3(nb), dim3(kCflThreads), 0,
-                               G.stream, f, e, x, dxs[0], dxs[1], dxs[2], dt, G.nint, partials, G.count, G.result);
+                               st, f, e, x, dxs[0], dxs[1], dxs[2], dt, G.nint, partials, G.count, G.result);
         else
             hipLaunchKernelGGL((k_icfl<decltype(NF)::value, decltype(D)::value, false>), dim3(nb), dim3(kCflThreads), 0,
-                               G.stream, f, e, x, dxs[0], dxs[1], dxs[2], dt, G.nint, partials, G.count, G.result);
+                               st, f, e, x, dxs[0], dxs[1], dxs[2], dt, G.nint, partials, G.count, G.result);
         HIPCHK(hipGetLastError());
         return 0;
     });
@@ -1493,12 +1500,13 @@ static int icfl_reduce(double *const *q, bool from_cons, double dt, double *out,
     // also reports errors.
     volatile uint64_t *r = (volatile uint64_t *)G.result;
     for (long n = 0; n < kPolls && *r == kPending; ++n) __builtin_ia32_pause();
-    if (*r == kPending) HIPCHK(hipStreamSynchronize(G.stream));
+    if (*r == kPending) HIPCHK(hipStreamSynchronize(st));
     *out = *(volatile double *)G.result;
     return 0;
 }
 
 int mfc_icfl_max(double *const *q_prim_vf, double dt, double *icfl_max) {
+    std::lock_guard<std::mutex> reduce(g_reduce);
     return icfl_reduce(q_prim_vf, false, dt, icfl_max, G.partials, kReduceBlocks, true);
 }
 
@@ -1506,6 +1514,7 @@ int mfc_stability_criteria(double *const *q_prim_vf, double dt, double *out) {
     if (!out) return fail(-1, "NULL output");
     out[1] = 0.0;
     out[2] = 0.0;
+    std::lock_guard<std::mutex> reduce(g_reduce);
     if (int rc = icfl_reduce(q_prim_vf, false, dt, &out[0], G.partials, kReduceBlocks, true)) return rc;
     if (!G.visc) return 0;
     Fields f;
@@ -1544,6 +1553,7 @@ static int cfl_dt(double *const *q_cons_vf, double cfl, double *dt_out, double *
     if (!(cfl > 0.0)) return fail(-1, "cfl must be positive");
     if (!dt_out) return fail(-1, "NULL output");
     double mx = 0.0;
+    std::lock_guard<std::mutex> reduce(g_reduce);
     if (int rc = icfl_reduce(q_cons_vf, true, 1.0, &mx, partials, kReduceBlocks, timed)) return rc;
     if (!(mx > 0.0) || mx != mx) return fail(-5, "CFL reduction gave %g (NaN or non-positive wave speed)", mx);
     *dt_out = cfl / mx;
