@@ -92,8 +92,9 @@ int mfc_rhs_init(const mfc_params *prm);
 /* In the forms other than MFC_PREC_FP64, a direction whose cells' WENO
  * coefficients all lie within 5e-13 (relative) of the first reconstructed
  * cell's (equal widths up to the rounding of the cell boundaries) is run
- * with the first cell's coefficients; MFC_PREC_FP64 does so only when they
- * are equal bit for bit. */
+ * with the first cell's coefficients, or in MFC_PREC_FP64_FAST with WENO5,
+ * where they also all lie within 5e-13 of the coefficients of equal widths,
+ * with those; MFC_PREC_FP64 does so only when they are equal bit for bit. */
 int mfc_rhs_set_grid(int dir, const double *s_cb, const double *ds);
 
 /* Replaces s_compute_rhs(q_cons_vf, q_prim_vf, rhs_vf, t_step)

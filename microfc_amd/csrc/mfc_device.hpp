@@ -50,6 +50,11 @@ struct Eos {
 // 18+3r+q.
 enum { kCbL = 0, kCbR = 6, kDL = 12, kDR = 15, kBeta = 18, kNCoef = 27 };
 
+// Kinds of WENO5 coefficients a kernel is built for: each cell's own from the
+// table; one set for every cell, in scalar registers; and in the contracted
+// form those of cells of equal width, built in (weno5_canon).
+enum CoefKind { kCellCoef = 0, kEqualCoef = 1, kCanonCoef = 2 };
+
 inline namespace MFC_FORM {
 
 constexpr bool kFastF64 = MFC_FAST_F64 != 0;
@@ -312,7 +317,7 @@ __device__ __forceinline__ void weno_cell(const R *v, const R *cf, R eps, R &vL,
 // from the cell value, one FMA each, and the cell value is added last, so
 // the rounding of the normalisation scales with the deviation instead of
 // with the value.  50 FP64 operations and a reciprocal instead of 62 in the
-// general form below; the sweeps are bound by VALU issue: 512^3 droplet x and
+// general form above; the sweeps are bound by VALU issue: 512^3 droplet x and
 // y sweep 9.13 -> 8.35 ms, z 5.59 -> 5.45 ms per launch, step 44.8 -> 42.1 ms,
 // 768^2 x and y sweep 47 -> 40 us.
 // The constants that are no inline operands are kept in scalar registers:
@@ -342,14 +347,16 @@ __device__ __forceinline__ void weno5_canon(const double *v, double eps, double 
     vR = __builtin_fma(nR, sL * r, v[2]);
 }
 
-// Both faces of one cell, as the uniform-grid (UNI) or per-cell kernels
-// reconstruct them.
-template <int WO, typename R, bool UNI>
+// Both faces of one cell, as the kernels of a coefficient kind (UNI, a
+// CoefKind) reconstruct them.
+template <int WO, typename R, int UNI>
 __device__ __forceinline__ void weno_both(const R *v, const R *cf, R eps, R &vL, R &vR, const CanonK &K) {
-    if constexpr (kFastF64 && sizeof(R) == 8 && WO == 5 && UNI)
+    if constexpr (UNI == kCanonCoef) {
+        static_assert(kFastF64 && sizeof(R) == 8 && WO == 5, "contracted form");
         weno5_canon(v, eps, vL, vR, K);
-    else
+    } else {
         weno_cell<WO, R, true, true>(v, cf, eps, vL, vR);
+    }
 }
 
 // HLLC flux at one face, normal direction DIR

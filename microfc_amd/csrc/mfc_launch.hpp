@@ -27,7 +27,7 @@ template <int NF, int FORM>
 int launch_sweep(const SweepLaunch &L, const SweepArgs &a, hipStream_t st);
 
 #define MFC_SWEEP_HELPERS(NF)                                                                           \
-    template <int D, int WO, typename R, bool ML, bool UNI>                                             \
+    template <int D, int WO, typename R, bool ML, int UNI>                                              \
     static int launch_nf##NF##_dwrm(int dir, const SweepArgs &a, hipStream_t st) {                      \
         const dim3 grid((unsigned)a.nblocks);                                                           \
         if (dir == 4) {                                                                                 \
@@ -54,10 +54,10 @@ int launch_sweep(const SweepLaunch &L, const SweepArgs &a, hipStream_t st);
             if constexpr (NF <= kXyMaxFluids && D >= 2 && WO == 5 && !ML && UNI) {                      \
                 if constexpr (D == 2 && sizeof(R) == 8)                                                 \
                     if (a.ghosts) {                                                                     \
-                        hipLaunchKernelGGL((k_sweep_xy<NF, D, R, true>), grid, dim3(kXyThreads), 0, st, a); \
+                        hipLaunchKernelGGL((k_sweep_xy<NF, D, R, true, UNI>), grid, dim3(kXyThreads), 0, st, a); \
                         return hipGetLastError() == hipSuccess ? 0 : -2;                                \
                     }                                                                                   \
-                hipLaunchKernelGGL((k_sweep_xy<NF, D, R, false>), grid, dim3(kXyThreads), 0, st, a);    \
+                hipLaunchKernelGGL((k_sweep_xy<NF, D, R, false, UNI>), grid, dim3(kXyThreads), 0, st, a);    \
             }                                                                                           \
             else return -1;                                                                             \
         } else if (dir == 0) {                                                                          \
@@ -75,9 +75,11 @@ int launch_sweep(const SweepLaunch &L, const SweepArgs &a, hipStream_t st);
     }                                                                                                   \
     template <int D, int WO, typename R>                                                                \
     static int launch_nf##NF##_dwr(int dir, const SweepArgs &a, hipStream_t st) {                       \
+        if constexpr (WO == 5 && kFastF64)                                                              \
+            if (a.uniform == kCanonCoef) return launch_nf##NF##_dwrm<D, 5, R, false, kCanonCoef>(dir, a, st); \
         if constexpr (WO == 5)                                                                          \
-            if (a.uniform) return launch_nf##NF##_dwrm<D, 5, R, false, true>(dir, a, st);               \
-        return launch_nf##NF##_dwrm<D, WO, R, false, false>(dir, a, st);                                \
+            if (a.uniform) return launch_nf##NF##_dwrm<D, 5, R, false, kEqualCoef>(dir, a, st);         \
+        return launch_nf##NF##_dwrm<D, WO, R, false, kCellCoef>(dir, a, st);                            \
     }                                                                                                   \
     template <int D, typename R>                                                                        \
     static int launch_nf##NF##_dr(const SweepLaunch &L, const SweepArgs &a, hipStream_t st) {           \
@@ -119,9 +121,9 @@ int launch_sweep(const SweepLaunch &L, const SweepArgs &a, hipStream_t st);
         if (L.precision == 2) {                                                                         \
             if (L.weno_order != 5) return -1;                                                           \
             switch (L.num_dims) {                                                                       \
-            case 1: return a.uniform ? launch_nf##NF##_dwrm<1, 5, float, true, true>(L.dir, a, st) : launch_nf##NF##_dwrm<1, 5, float, true, false>(L.dir, a, st);                       \
-            case 2: return a.uniform ? launch_nf##NF##_dwrm<2, 5, float, true, true>(L.dir, a, st) : launch_nf##NF##_dwrm<2, 5, float, true, false>(L.dir, a, st);                       \
-            case 3: return a.uniform ? launch_nf##NF##_dwrm<3, 5, float, true, true>(L.dir, a, st) : launch_nf##NF##_dwrm<3, 5, float, true, false>(L.dir, a, st);                       \
+            case 1: return a.uniform ? launch_nf##NF##_dwrm<1, 5, float, true, kEqualCoef>(L.dir, a, st) : launch_nf##NF##_dwrm<1, 5, float, true, kCellCoef>(L.dir, a, st);              \
+            case 2: return a.uniform ? launch_nf##NF##_dwrm<2, 5, float, true, kEqualCoef>(L.dir, a, st) : launch_nf##NF##_dwrm<2, 5, float, true, kCellCoef>(L.dir, a, st);              \
+            case 3: return a.uniform ? launch_nf##NF##_dwrm<3, 5, float, true, kEqualCoef>(L.dir, a, st) : launch_nf##NF##_dwrm<3, 5, float, true, kCellCoef>(L.dir, a, st);              \
             default: return -1;                                                                         \
             }                                                                                           \
         }                                                                                               \

@@ -132,7 +132,7 @@ constexpr int march_waves() { return sizeof(R) == 4 ? 3 : 2; }
 // right-hand side whose caller asks for them; the ghost cells' come from
 // k_bc_prim).  A pass of its own read the state for it: 256^3 cells 3.24 ->
 // 2.91 ms with it stored here, 1400 x 1300 251 -> 225 us.
-template <int NF, int D, int MD, typename R, bool WX, bool UNI, bool PO = false>
+template <int NF, int D, int MD, typename R, bool WX, int UNI, bool PO = false>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(march_waves<R>(), march_waves<R>()))) void k_march(const SweepArgs a) {
     static_assert((MD == 1 && WX) || (!WX && D == 3), "y march with the x faces, y and z march");
     using Y = Sys<NF, D>;
@@ -144,7 +144,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(march_waves<
     constexpr int HL = WX ? PN : 0;            // ring entries before lane 0's
     constexpr int RW = 64 + 2 * HL;            // entries of a ring row
     constexpr int HB = sizeof(R) == 8 ? 4 : 8; // rows per batch of the entries around the lanes'
-    constexpr bool CANON = kFastF64 && sizeof(R) == 8 && UNI;
+    constexpr bool CANON = UNI == kCanonCoef;
     // the RK base: the z march adds the first kBaseOnZFused variables
     constexpr int BLO = MD == 1 && D == 3 ? kBaseOnZFused : 0, BHI = MD == 1 ? S : kBaseOnZFused;
     // whether rhs holds another direction's part: in 3D the sums begin in the

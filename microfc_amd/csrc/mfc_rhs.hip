@@ -74,7 +74,9 @@ constexpr int kBaseOnZ = 4;
 // inside the contracted form's 1e-12.  The plain FP64 form keeps the
 // per-cell coefficients unless they are equal bit for bit.
 constexpr double kUniformRelTol = 5e-13;
-// WENO5 coefficients of cells of equal width (plane order of mfc_device.hpp).
+// WENO5 coefficients of cells of equal width (plane order of mfc_device.hpp):
+// what the contracted form runs with where every cell lies within
+// kUniformRelTol of them too.
 constexpr double kCanon[kNCoef] = {
     1.0 / 3, -5.0 / 6, -1.0 / 6, -1.0 / 3, -2.0 / 3, 1.0 / 6, -1.0 / 6, 2.0 / 3,   1.0 / 3,
     1.0 / 6, 5.0 / 6,  -1.0 / 3, 0.1,      0.6,      0.3,     0.3,      0.6,       0.1,
@@ -135,6 +137,9 @@ struct Dir {
     // every reconstructed cell has the same coefficients: bit for bit in the
     // plain FP64 form, to kUniformRelTol in the others
     bool uniform = false;
+    // contracted form, WENO5: uniform, and every reconstructed cell's
+    // coefficients within kUniformRelTol of equal widths' (kCanon)
+    bool canon = false;
     double ucf[kNCoef] = {};
     bool uniform_wide = false; // the same over every cell the coefficients are set for (-b+polyn..s+b-polyn)
 };
@@ -794,6 +799,11 @@ int cons_to_prim_launch(const Fields &qc, const Fields &qp) {
     });
 }
 
+// The coefficients (a CoefKind) that a kernel of directions d and e has.
+int coef_kind(int d, int e) {
+    return G.dir[d].canon && G.dir[e].canon ? kCanonCoef : G.dir[d].uniform && G.dir[e].uniform ? kEqualCoef : kCellCoef;
+}
+
 SweepArgs sweep_args(int d) {
     SweepArgs a;
     memset(&a, 0, sizeof a);
@@ -815,7 +825,7 @@ SweepArgs sweep_args(int d) {
     a.bc_beg = bcs[d][0];
     a.bc_end = bcs[d][1];
     memcpy(a.bcs, bcs, sizeof bcs);
-    a.uniform = G.dir[d].uniform ? 1 : 0;
+    a.uniform = coef_kind(d, d);
     for (int q = 0; q < kNCoef; ++q) {
         a.ucf[q] = G.dir[d].ucf[q];
         a.ucf32[q] = (float)G.dir[d].ucf[q];
@@ -855,6 +865,7 @@ SweepArgs sweep_args(int d) {
 // direction's cell widths, boundary codes and coefficients, and its tiles.
 SweepArgs xy_args() {
     SweepArgs a = sweep_args(0);
+    a.uniform = coef_kind(0, 1);
     a.inv_ds2 = G.dir[1].inv_ds;
     a.bc2_beg = G.prm.bc_y_beg;
     a.bc2_end = G.prm.bc_y_end;
@@ -877,7 +888,6 @@ SweepArgs march_args(int d) {
     if (d == 4) {
         a.coef2 = G.dir[1].coef;
         a.ncell2 = G.dir[1].s + 2 * G.b + 1;
-        a.uniform = G.dir[0].uniform && G.dir[1].uniform;
     }
     a.rl = d == 4 ? G.prm.m + 1 + 2 * kMarchHaloXY : G.prm.m + 1;
     a.ntile = (int)(((long)a.rl * other + cells - 1) / cells);
@@ -958,7 +968,6 @@ SweepArgs stage_args() {
     if (G.D == 2) {
         a.coef2 = G.dir[1].coef;
         a.ncell2 = G.dir[1].s + 2 * G.b + 1;
-        a.uniform = G.dir[0].uniform && G.dir[1].uniform;
     }
     a.ntile = (G.prm.m + stage_cells_x(G.D)) / stage_cells_x(G.D);
     a.nblocks = (long)a.ntile * ((G.prm.n + stage_cells_y(G.D)) / stage_cells_y(G.D));
@@ -1310,7 +1319,8 @@ int mfc_rhs_set_grid(int dir, const double *s_cb, const double *ds) {
     weno_tables(s, b, G.prm.weno_order, s_cb, D.coef_h);
     // Uniform coefficients over the cells the sweeps reconstruct (-1..s+1)?
     // Bit for bit in the plain FP64 form; within kUniformRelTol of cell -1's
-    // in the others, whose uniform-grid kernels then use cell -1's.
+    // in the others, whose uniform-grid kernels then use cell -1's (but see
+    // canon).
     {
         const long nc = s + 2 * b + 1;
         const double tol = G.prm.precision == MFC_PREC_FP64 ? 0.0 : kUniformRelTol;
@@ -1324,14 +1334,18 @@ int mfc_rhs_set_grid(int dir, const double *s_cb, const double *ds) {
             }
         }
     }
-    // The contracted form's uniform-grid WENO5 kernels have the constants of
-    // equal cell widths built in (weno5_canon): equal coefficients of unequal
-    // widths (a geometric grid) run the per-cell kernels.
-    if (G.prm.precision == MFC_PREC_FP64_FAST && G.prm.weno_order == 5)
-        for (int q = 0; q < kNCoef && D.uniform; ++q)
-            D.uniform = std::fabs(D.ucf[q] - kCanon[q]) <= kUniformRelTol * std::fabs(kCanon[q]);
-    // ... and over every cell with coefficients (the weno_Re_flux gradient
-    // pass reconstructs the ghost cells too)
+    // The contracted form has WENO5 kernels with the constants of equal cell
+    // widths built in (weno5_canon), for cells that all lie within the same
+    // tolerance of those.  Equal coefficients of unequal widths (a geometric
+    // grid) keep cell -1's: with each cell's own, 1024^2 cells took 311 instead
+    // of 234 us per step, 64^3 204 instead of 170.
+    D.canon = D.uniform && G.prm.precision == MFC_PREC_FP64_FAST && G.prm.weno_order == 5;
+    for (int q = 0; q < kNCoef && D.canon; ++q)
+        for (int j = -1; j <= s + 1 && D.canon; ++j)
+            D.canon = std::fabs(D.coef_h[(long)q * (s + 2 * b + 1) + (j + b)] - kCanon[q]) <=
+                      kUniformRelTol * std::fabs(kCanon[q]);
+    // Uniform over every cell with coefficients (the weno_Re_flux gradient
+    // pass reconstructs the ghost cells too)?
     {
         const long nc = s + 2 * b + 1;
         const int pn = (G.prm.weno_order - 1) / 2;

@@ -76,7 +76,7 @@ __device__ __forceinline__ void store_ghosts_of(const SweepArgs &a, double *q, i
 // own clock (2D, per-cell coefficients): loads 2.1 us, conversion 0.6,
 // reconstruction 4.4, faces 1.9, finish 1.2.  Coefficients loaded per wave
 // instead of per block cost 1.4 us more.
-template <int NF, int D, bool UNI>
+template <int NF, int D, int UNI>
 __global__ __launch_bounds__(stage_threads(NF, D)) void k_stage(const SweepArgs a) {
     using L = StageTile<NF, D>;
     using Y = Sys<NF, D>;

@@ -80,7 +80,7 @@ struct SweepArgs {
     const MlpFrags *mlp;  // learned WENO5 weights (MFC_PREC_FP32_LEARNED)
     // Uniform grids: when every cell the sweep reconstructs has the same 27
     // coefficients (bit for bit), they travel here as kernel arguments (read
-    // into scalar registers) instead of being loaded per cell.
+    // into scalar registers) instead of being loaded per cell (a CoefKind).
     int uniform;
     double ucf[kNCoef];
     float ucf32[kNCoef];
@@ -535,7 +535,7 @@ __device__ __forceinline__ void load_cons_prim(const SweepArgs &a, long go, doub
     cons_to_prim<NF, D>(c, p, a.eos);
 }
 
-template <typename R, int WO, bool UNI>
+template <typename R, int WO, int UNI>
 __device__ __forceinline__ void load_coef(const SweepArgs &a, int cell, R *cf) {
     if constexpr (WO > 1 && UNI) {
 #pragma unroll
@@ -670,9 +670,9 @@ __device__ __forceinline__ void ml_face_states(int var, const float *stR, const 
 // cell-parallel is 6 % faster in FP32 and with uniform FP64 coefficients,
 // and no faster for FP64 with per-cell coefficient loads, whose registers
 // then cost a wave of occupancy.
-template <bool ML, typename R, bool UNI>
+template <bool ML, typename R, int UNI>
 constexpr bool x_cell_parallel() { return ML || sizeof(R) == 4 || UNI; }
-template <bool ML, typename R, bool UNI>
+template <bool ML, typename R, int UNI>
 constexpr int x_tile_cells() { return x_cell_parallel<ML, R, UNI>() ? 62 : 63; }
 
 // Whether the x sweep, where it writes an RK stage, fills the stage's ghost
@@ -683,7 +683,7 @@ constexpr int x_tile_cells() { return x_cell_parallel<ML, R, UNI>() ? 62 : 63; }
 // to k_bc_fill, and so does 3D, where a corner cell has 124 copies.
 constexpr bool x_fills_ghosts(int D, bool ml) { return D == 1 || (ml && D == 2); }
 
-template <int NF, int D, int WO, typename R, bool ML, bool UNI>
+template <int NF, int D, int WO, typename R, bool ML, int UNI>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(ML ? 2 : 4, 8))) void k_sweep_x(const SweepArgs a) {
     using Y = Sys<NF, D>;
     constexpr int S = Y::S;
@@ -921,7 +921,7 @@ constexpr int t_faces() { return 16; }
 template <bool ML>
 constexpr int t_threads() { return kTX * t_faces<ML>(); }
 // The y/z sweep is cell-parallel (k_sweep_tc) in the forms whose x sweep is.
-template <bool ML, typename R, bool UNI>
+template <bool ML, typename R, int UNI>
 constexpr bool t_cell_parallel() { return x_cell_parallel<ML, R, UNI>(); }
 // Threads per column of the cell-parallel tile (a power of two <= 64; the
 // column's lanes are consecutive within a wave): tc_rows_of (plain and
@@ -930,12 +930,12 @@ template <typename R>
 constexpr int tc_rows(int dir) { return tc_rows_of(sizeof(R) == 8, kFastF64, dir); }
 template <typename R, bool ML>
 constexpr int tc_cols(int dir) { return tc_cols_of(ML, dir); }
-template <bool ML, typename R, bool UNI>
+template <bool ML, typename R, int UNI>
 constexpr int t_tile_cells(int dir) {
     return t_cell_parallel<ML, R, UNI>() ? tc_rows<R>(dir) - 2 : t_faces<ML>() - 1;
 }
 
-template <int NF, int D, int DIR, int WO, typename R, bool ML, bool UNI>
+template <int NF, int D, int DIR, int WO, typename R, bool ML, int UNI>
 __global__ __launch_bounds__(t_threads<ML>()) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_sweep_t(
     const SweepArgs a) {
     static_assert(!ML, "the learned form runs the cell-parallel sweep");
@@ -1113,7 +1113,7 @@ __device__ __forceinline__ R row_next(R x) {
     return __shfl_down(x, 1u, W);
 }
 
-template <int NF, int D, int DIR, int WO, typename R, bool ML, bool UNI>
+template <int NF, int D, int DIR, int WO, typename R, bool ML, int UNI>
 __global__ __launch_bounds__((tc_cols<R, ML>(DIR) * tc_rows<R>(DIR)))
     __attribute__((amdgpu_waves_per_eu(ML ? 2 : 4, 8))) void k_sweep_tc(const SweepArgs a) {
     static_assert(t_cell_parallel<ML, R, UNI>(), "cell-parallel forms only");
@@ -1425,7 +1425,7 @@ __device__ __forceinline__ void xy_halo_cell(int h, int &cx, int &ry) {
 
 // GH: fills the stage output's ghost cells (store_ghosts; 2D FP64: 768^2
 // contracted 194 -> 176 us per step with its CFL reduction).
-template <int NF, int D, typename R, bool GH>
+template <int NF, int D, typename R, bool GH, int UNI>
 __global__ __launch_bounds__(kXyThreads) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_sweep_xy(const SweepArgs a) {
     static_assert(sizeof(R) == 8 || sizeof(R) == 4, "FP64 or FP32 reconstruction");
     using Y = Sys<NF, D>;
@@ -1515,7 +1515,7 @@ __global__ __launch_bounds__(kXyThreads) __attribute__((amdgpu_waves_per_eu(4, 8
             R st[5], vl;
 #pragma unroll
             for (int w = 0; w < 5; ++w) st[w] = sp[v][cx][yr + w];
-            weno_both<5, R, true>(st, cf, eps, vl, qL[v], CanonK());
+            weno_both<5, R, UNI>(st, cf, eps, vl, qL[v], CanonK());
             qR[v] = __shfl_down(vl, 1u, YK);
         }
         const int jf = y0 - 1 + yr;
@@ -1543,7 +1543,7 @@ __global__ __launch_bounds__(kXyThreads) __attribute__((amdgpu_waves_per_eu(4, 8
             R st[5], vl;
 #pragma unroll
             for (int w = 0; w < 5; ++w) st[w] = sp[v][c + w][ry];
-            weno_both<5, R, true>(st, cf, eps, vl, qL[v], CanonK());
+            weno_both<5, R, UNI>(st, cf, eps, vl, qL[v], CanonK());
             qR[v] = __shfl_down(vl, 1u, XL);
         }
         const int jf = x0 - 1 + c;
