@@ -82,9 +82,19 @@ constexpr double kCanon[kNCoef] = {
     1.0 / 6, 5.0 / 6,  -1.0 / 3, 0.1,      0.6,      0.3,     0.3,      0.6,       0.1,
     4.0 / 3, -11.0 / 3, 10.0 / 3, 4.0 / 3, -5.0 / 3, 4.0 / 3, 10.0 / 3, -11.0 / 3, 4.0 / 3};
 constexpr bool kFuseXY = true;
-// Waves of a march the chip runs at a time (8 per CU), and the fewest rows of
-// a chunk.
-constexpr int kMarchSlots = 8 * 256, kMarchRowsMin = 16;
+// Waves of a march in FP64 and in FP32 (march_waves), or of k_rows_x, that the
+// chip runs at a time; the fewest rows of a grid that marches, and of a chunk.
+constexpr int kMarchSlots = 8 * 256, kMarchSlots32 = 12 * 256, kMarchRowsMin = 16, kMarchChunkMin = 8;
+// The time of `waves` of a march on so many slots, in times of one: one round
+// as long as all have a place at once, else the last round is half empty.  With
+// that half round added throughout and 16 rows the least of a chunk, a few waves
+// were left for a second round: FP32 bulk on unequal widths 115^3 904 -> 722,
+// 120^3 1005 -> 804 us per step (800 and 909 in the separate sweeps), plain 4096
+// x 2048 2725 -> 2596 (2605 in the tiles).
+double chunk_rounds(double waves, int slots) {
+    const double r = waves / slots;
+    return r <= 1.0 ? 1.0 : r + 0.5;
+}
 // Cells from which a march (k_march) takes over, where both were measured
 // (ms per RK3 step, tile kernels -> marches; two fluids):
 //  * equal widths, 3D: contracted FP64 128^3 0.82 -> 0.82, 200^3 2.72 -> 2.63,
@@ -102,7 +112,13 @@ constexpr int kMarchSlots = 8 * 256, kMarchRowsMin = 16;
 //    contracted 150 x 112 x 92 1.38 -> 1.12, 180 x 130 x 90 1.79 -> 1.40; plain
 //    150 x 112 x 92 1.86 -> 1.60; FP32 bulk 200^3, z alone 4.93 -> 4.81 (with y
 //    4.88); equal widths 256^3, z alone: contracted 8.70 -> 8.26 (with y 8.41),
-//    plain 14.3 -> 13.7.
+//    plain 14.3 -> 13.7;
+//  * just above these lines, with the chunks of chunk_rounds: equal widths 4096
+//    x 2048 contracted 1.67 -> 1.28, plain 2.61 -> 2.54 (one fluid 2.09 -> 2.00);
+//    other widths 1300^2 contracted 0.570 -> 0.361, plain 0.755 -> 0.638, FP32
+//    bulk 0.478 -> 0.376 (one fluid 0.318 -> 0.293); 120^3 contracted 1.08 ->
+//    0.73, plain 1.43 -> 1.18, FP32 bulk 0.909 -> 0.803 (one fluid 0.675 ->
+//    0.559).
 // The FP32-bulk form on equal widths keeps its tiles (300 x 250 x 200 4.75 ->
 // 4.91): with half the LDS and registers they fill the SIMDs already.
 constexpr double kMarchUniform2D = 8e6, kMarchUniform3D = 3e6, kMarchPerCell = 1.5e6;
@@ -892,15 +908,14 @@ SweepArgs march_args(int d) {
     a.rl = d == 4 ? G.prm.m + 1 + 2 * kMarchHaloXY : G.prm.m + 1;
     a.ntile = (int)(((long)a.rl * other + cells - 1) / cells);
     // Chunks of rows: a chunk costs three rows more than it finishes (the
-    // staged rows and the reconstructions before its first face), and the
-    // chip runs kMarchSlots waves at a time, the last round half empty.
+    // staged rows and the reconstructions before its first face).
+    const int slots = G.prm.precision == MFC_PREC_FP32_BULK ? kMarchSlots32 : kMarchSlots;
     double best = 0.0;
     for (int nc = 1; nc <= rows; ++nc) {
         const int L = (rows + nc - 1) / nc;
-        if (L < kMarchRowsMin && nc > 1) break;
+        if (L < kMarchChunkMin && nc > 1) break;
         if ((rows + L - 1) / L != nc) continue;
-        const double rounds = std::max(1.0, (double)a.ntile * nc / kMarchSlots + 0.5);
-        const double cost = rounds * (L + 3);
+        const double cost = chunk_rounds((double)a.ntile * nc, slots) * (L + 3);
         if (best == 0.0 || cost < best) best = cost, a.chunk = L, a.nchunk = nc;
     }
     a.nblocks = (long)a.ntile * a.nchunk;
@@ -923,9 +938,9 @@ bool marches(int d) {
     // short rows or few of them: the lanes and rows a march adds at the ends
     // would outweigh what it saves
     const SweepArgs a = march_args(d);
-    return a.chunk >= kMarchRowsMin &&
-           (double)G.nint / (d == 5 ? G.prm.p + 1 : G.prm.n + 1) >=
-               0.85 * a.ntile * (d == 4 ? kMarchCellsXY : kMarchCellsZ);
+    const int rows = d == 5 ? G.prm.p + 1 : G.prm.n + 1;
+    return rows >= kMarchRowsMin &&
+           (double)G.nint / rows >= 0.85 * a.ntile * (d == 4 ? kMarchCellsXY : kMarchCellsZ);
 }
 
 // Arguments of k_rows_x.
