@@ -948,13 +948,17 @@ SweepArgs rows_args() {
     SweepArgs a = sweep_args(0);
     a.rl = G.prm.m + 7;
     a.ntile = (int)(((long)a.rl * (G.prm.p + 1) + kRowsCells - 4) / kRowsCells);
-    // chunks as in march_args; a chunk costs about a row more than it finishes
-    // (the coefficients' loads)
+    // Chunks as in march_args; a chunk costs about half a row more than it
+    // finishes (the coefficients' loads).  Past one round the launch's time
+    // grows in half rounds, one wave more per SIMD each (16 grids with 1 to 13
+    // rows a chunk: 1.41 rounds' time for 1.06 rounds of waves, 1.47 for 1.49,
+    // 1.85 for 1.59, 2.32 for 2.22).
     const int rows = G.prm.n + 1;
     double best = 0.0;
     for (int L = 1; L <= std::min(rows, 32); ++L) {
         const int nc = (rows + L - 1) / L;
-        const double cost = std::max(1.0, (double)a.ntile * nc / kMarchSlots + 0.5) * (L + 1);
+        const double r = (double)a.ntile * nc / kMarchSlots;
+        const double cost = (r <= 1.0 ? 1.0 : 0.1 + 0.45 * std::ceil(2.0 * r)) * (L + 0.5);
         if (best == 0.0 || cost < best) best = cost, a.chunk = L, a.nchunk = nc;
     }
     a.nblocks = (long)a.ntile * a.nchunk;
@@ -962,19 +966,21 @@ SweepArgs rows_args() {
 }
 
 // Whether the x direction of a case on unequal widths runs along rows
-// (k_rows_x): from two rounds of waves with a row each.  RK3 step, plain or
-// contracted (c), x sweep -> rows: 400 x 300 cells (2400 sets of columns and
-// rows) 106 -> 104 us, 600 x 500 (5500) 185 -> 180, 700 x 700 269 -> 247, 1000 x
-// 900 428 -> 397, c 800 x 800 219 -> 211; 70 x 60 x 60 (4800) 340 -> 287, 96^3
-// 804 -> 750, but c 60 x 56 x 50 (3300) 155 -> 156; three fluids c 60 x 50 x 40
-// 156 -> 162, 180 x 130 x 90 1436 -> 1284, plain 2080 -> 1990.
-constexpr long kRowsMin = 2 * kMarchSlots;
+// (k_rows_x): from two rounds of waves with a row each, and where the x sweep's
+// waves (63 cells each, four per SIMD) do not all have a place at once.  RK3
+// step, plain or contracted (c), x sweep -> rows: 600 x 500 cells (5500 sets of
+// columns and rows) 188 -> 179 us, 700 x 700 269 -> 245, 1000 x 900 411 -> 388, c
+// 800 x 800 214 -> 205; 96^3 750 -> 696; three fluids c 180 x 130 x 90 1806 ->
+// 1221, plain 2349 -> 1841.  Just above the line 64 x 69 x 51 (4278 sets, 7038
+// waves of the x sweep; RK2) 210 -> 178; where the x sweep has fewer than 4096
+// waves rows took 0.97 to 1.06 of its time (57 x 82 x 48 185 -> 191).
+constexpr long kRowsMin = 2 * kMarchSlots, kSweepXSlots = 16 * 256;
 bool rows_x() {
     if (G.D < 2 || G.visc || G.prm.weno_order != 5 || G.prm.num_fluids > kRowsMaxFluids || G.dir[0].uniform ||
         (G.prm.precision != MFC_PREC_FP64 && G.prm.precision != MFC_PREC_FP64_FAST))
         return false;
     if (G.ng * (long)sizeof(double) >= (1L << 32)) return false; // 32-bit byte offsets within a variable
-    return (long)rows_args().ntile * (G.prm.n + 1) >= kRowsMin;
+    return sweep_args(0).nblocks > kSweepXSlots && (long)rows_args().ntile * (G.prm.n + 1) >= kRowsMin;
 }
 
 // Arguments of k_stage.
