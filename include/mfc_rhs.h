@@ -210,7 +210,10 @@ const char *mfc_mlp_last_error(void);
  * 4 sweep_z, 5 icfl, 6 rk1_update, 7 viscous (the gradient pass or one
  * direction of a viscous run), 8 sweep_xy (x and y together: the fused tile,
  * the march of large grids, or the whole RK stage of a small 2D case; a small
- * 1D case's stage counts as sweep_x).  The reference's only timing is the mean
+ * 1D case's stage counts as sweep_x).  Which kernel a sweep was is counted
+ * once more under 9 tile_xy (the fused tile), 10 march_xy, 11 march_z, 12
+ * march_y, 13 rows_x (x along rows) and 14 stage (a whole RK stage); the sweeps
+ * counted under none of these are the separate ones.  The reference's only timing is the mean
  * CPU time per step (src/simulation/m_time_steppers.fpp:281,352-358). */
 int mfc_timing_enable(int on);
 int mfc_timing_reset(void);

@@ -180,14 +180,17 @@ struct State {
 
 // ---------------------------------------------------------------------------
 // Optional per-kernel timing with HIP events on the library's stream.
-enum KernelId { kKBcFill = 0, kKConsToPrim, kKSweepX, kKSweepY, kKSweepZ, kKIcfl, kKRk1, kKViscous, kKSweepXY, kKCount };
+enum KernelId { kKBcFill = 0, kKConsToPrim, kKSweepX, kKSweepY, kKSweepZ, kKIcfl, kKRk1, kKViscous, kKSweepXY,
+                // which kernel a sweep was, counted beside its direction's id
+                kKTileXY, kKMarchXY, kKMarchZ, kKMarchY, kKRowsX, kKStage, kKCount };
 const char *const kKernelNames[kKCount] = {"bc_fill", "cons_to_prim", "sweep_x", "sweep_y", "sweep_z", "icfl",
-                                           "rk1_update", "viscous", "sweep_xy"};
+                                           "rk1_update", "viscous", "sweep_xy", "tile_xy", "march_xy", "march_z",
+                                           "march_y", "rows_x", "stage"};
 
 struct Timing {
     bool on = false;
     struct Rec {
-        int id;
+        int id, sub;
         hipEvent_t a, b;
     };
     std::vector<Rec> pending;
@@ -207,9 +210,9 @@ struct Timing {
 } T;
 
 struct TimedScope {
-    int id;
+    int id, sub;
     hipEvent_t a = nullptr;
-    explicit TimedScope(int k) : id(k) { // k < 0: not timed
+    explicit TimedScope(int k, int s = -1) : id(k), sub(s) { // k < 0: not timed; s >= 0: counted there too
         if (k >= 0 && T.on && (a = T.get())) (void)hipEventRecord(a, G.stream);
     }
     ~TimedScope() {
@@ -217,7 +220,7 @@ struct TimedScope {
         hipEvent_t b = T.get();
         if (!b) return;
         (void)hipEventRecord(b, G.stream);
-        T.pending.push_back({id, a, b});
+        T.pending.push_back({id, sub, a, b});
     }
 };
 
@@ -227,8 +230,11 @@ int timing_flush() {
     for (auto &r : T.pending) {
         float ms = 0.f;
         HIPCHK(hipEventElapsedTime(&ms, r.a, r.b));
-        T.total_ms[r.id] += ms;
-        T.count[r.id] += 1;
+        for (int k : {r.id, r.sub})
+            if (k >= 0) {
+                T.total_ms[k] += ms;
+                T.count[k] += 1;
+            }
         T.pool.push_back(r.a);
         T.pool.push_back(r.b);
     }
@@ -1017,7 +1023,8 @@ int sweep(int d, SweepArgs &a) {
     }
     static constexpr int kinds[] = {kKSweepX, kKSweepX + 1, kKSweepX + 2, kKSweepXY, kKSweepXY, kKSweepZ, kKSweepXY,
                                     kKSweepX + 1, kKSweepX};
-    TimedScope ts(d == 6 && G.D == 1 ? kKSweepX : kinds[d]);
+    static constexpr int subs[] = {-1, -1, -1, kKTileXY, kKMarchXY, kKMarchZ, kKStage, kKMarchY, kKRowsX};
+    TimedScope ts(d == 6 && G.D == 1 ? kKSweepX : kinds[d], subs[d]);
     int rc;
     const int form = G.prm.precision == MFC_PREC_FP64        ? kFormF64
                      : G.prm.precision == MFC_PREC_FP64_FAST ? kFormF64Fast

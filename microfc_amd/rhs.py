@@ -42,6 +42,8 @@ EXPORTED = [
 ]
 KERNEL_IDS = {"bc_fill": 0, "cons_to_prim": 1, "sweep_x": 2, "sweep_y": 3, "sweep_z": 4, "icfl": 5,
               "rk1_update": 6, "viscous": 7, "sweep_xy": 8}
+# which kernel a sweep was, counted beside the ids above
+VARIANT_IDS = {"tile_xy": 9, "march_xy": 10, "march_z": 11, "march_y": 12, "rows_x": 13, "stage": 14}
 
 
 class MfcError(RuntimeError):
@@ -351,8 +353,16 @@ class RhsModule:
             _check(self.lib.mfc_timing_reset(), "mfc_timing_reset")
         if enable is not None:
             _check(self.lib.mfc_timing_enable(1 if enable else 0), "mfc_timing_enable")
+        return self._timing_of(KERNEL_IDS)
+
+    def timing_variants(self):
+        """{name: launches} of the sweeps' kernels (include/mfc_rhs.h) since the
+        last reset, while timing was on; those not launched are left out."""
+        return {k: v[1] for k, v in self._timing_of(VARIANT_IDS).items() if v[1]}
+
+    def _timing_of(self, ids):
         out = {}
-        for name, k in KERNEL_IDS.items():
+        for name, k in ids.items():
             nm = ctypes.c_char_p()
             ms = ctypes.c_double()
             cnt = ctypes.c_long()
