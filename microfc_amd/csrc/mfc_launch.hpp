@@ -39,13 +39,13 @@ int launch_sweep(const SweepLaunch &L, const SweepArgs &a, hipStream_t st);
             if constexpr (NF <= kMarchMaxFluidsXY && D >= 2 && WO == 5 && !ML && (sizeof(R) == 8 || !UNI)) hipLaunchKernelGGL((k_march<NF, D, 1, R, true, UNI>), grid, dim3(64), 0, st, a); \
             else return -1;                                                                             \
         } else if (dir == 5) {                                                                          \
-            if constexpr (NF <= kMarchMaxFluidsZ && D == 3 && WO == 5 && !ML) hipLaunchKernelGGL((k_march<NF, 3, 2, R, false, UNI>), grid, dim3(64), 0, st, a); \
+            if constexpr (NF <= kMarchMaxFluidsZ && D == 3 && WO == 5 && !ML && (sizeof(R) == 8 || !UNI)) hipLaunchKernelGGL((k_march<NF, 3, 2, R, false, UNI>), grid, dim3(64), 0, st, a); \
             else return -1;                                                                             \
         } else if (dir == 8) {                                                                          \
             if constexpr (NF <= kRowsMaxFluids && D >= 2 && WO == 5 && !ML && !UNI && sizeof(R) == 8) hipLaunchKernelGGL((k_rows_x<NF, D>), grid, dim3(64), 0, st, a); \
             else return -1;                                                                             \
         } else if (dir == 7) {                                                                          \
-            if constexpr (NF > kMarchMaxFluidsXY && NF <= kMarchMaxFluidsZ && D == 3 && WO == 5 && !ML) hipLaunchKernelGGL((k_march<NF, 3, 1, R, false, UNI>), grid, dim3(64), 0, st, a); \
+            if constexpr (NF > kMarchMaxFluidsXY && NF <= kMarchMaxFluidsZ && D == 3 && WO == 5 && !ML && sizeof(R) == 8 && !UNI) hipLaunchKernelGGL((k_march<NF, 3, 1, R, false, UNI>), grid, dim3(64), 0, st, a); \
             else return -1;                                                                             \
         } else if (dir == 6) {                                                                          \
             if constexpr (NF <= kXyMaxFluids && D <= 2 && WO == 5 && !ML && sizeof(R) == 8) hipLaunchKernelGGL((k_stage<NF, D, UNI>), grid, dim3(stage_threads(NF, D)), 0, st, a); \

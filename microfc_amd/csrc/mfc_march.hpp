@@ -135,6 +135,7 @@ constexpr int march_waves() { return sizeof(R) == 4 ? 3 : 2; }
 template <int NF, int D, int MD, typename R, bool WX, int UNI, bool PO = false>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(march_waves<R>(), march_waves<R>()))) void k_march(const SweepArgs a) {
     static_assert((MD == 1 && WX) || (!WX && D == 3), "y march with the x faces, y and z march");
+    static_assert(sizeof(R) == 8 || !UNI, "FP32 marches are for unequal widths");
     using Y = Sys<NF, D>;
     constexpr int S = Y::S;
     constexpr int PN = 2;
@@ -313,8 +314,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(march_waves<
                     if constexpr (UNI) {
 #pragma unroll
                         for (int c = 0; c < kNCoef; ++c)
-                            cf[c] = WX ? (sizeof(R) == 8 ? (R)b.ucf2[c] : (R)b.ucf2_32[c])
-                                       : (sizeof(R) == 8 ? (R)b.ucf[c] : (R)b.ucf32[c]);
+                            cf[c] = WX ? b.ucf2[c] : b.ucf[c];
                     } else {
                         const double *tab = WX ? b.coef2 : b.coef;
                         const long nc = WX ? b.ncell2 : b.ncell;
@@ -364,7 +364,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(march_waves<
                         march_prim_in<NF, D, R, FM>(args(), pv, fin);
                     }
                     if (finish)
-                        finish_cell<NF, D, R, FM, false>(args(), go, ro, a.inv_ds[jr], fl, f, usl, us, fin, BLO, BHI, x, t, jr);
+                        finish_cell<NF, D, R, FM, false>(args(), go, ro, a.inv_ds[jr], fl, f, usl, us, fin, BLO, BHI, x, t);
                 } else {
                     // 2. x faces of row jr
                     const double iy = a.inv_ds2[jr];
@@ -388,7 +388,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(march_waves<
                         R qL[S], qR[S], cf[kNCoef];
                         if constexpr (!CANON && UNI) {
 #pragma unroll
-                            for (int c = 0; c < kNCoef; ++c) cf[c] = sizeof(R) == 8 ? (R)b.ucf[c] : (R)b.ucf32[c];
+                            for (int c = 0; c < kNCoef; ++c) cf[c] = b.ucf[c];
                         }
                         R nx[5];
 #pragma unroll
@@ -429,7 +429,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(march_waves<
                     for (int v = 0; v < NK; ++v) fin.in[Y::MOM + v] = ko[v];
                     if (finish) march_prim_in<NF, D, R, FM>(args(), w0, fin);
                     if (finish)
-                        finish_xy<NF, D, R, false>(args(), fresh_args(), go, ro, ix, iy, dfx, dux, duy, fin, x, jr, t,
+                        finish_xy<NF, D, R, false>(args(), fresh_args(), go, ro, ix, iy, dfx, dux, duy, fin, x, jr,
                                             [&](int v, bool, double) { return acc[v]; });
                 }
             }

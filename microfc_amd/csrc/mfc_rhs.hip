@@ -1056,11 +1056,10 @@ int sweep(int d, SweepArgs &a) {
 // Direction d of a viscous RHS evaluation (inviscid and viscous fluxes of
 // every face, then the finish: m_rhs.fpp:565-652), with sa the direction's
 // finish arguments (rhs assignment or accumulation, or the RK stage).
-int viscous(int d, const Fields &qin, const Fields &rhs, const SweepArgs &sa) {
+int viscous(int d, const Fields &qin, const SweepArgs &sa) {
     ViscArgs v;
     memset(&v, 0, sizeof v);
     v.q = qin;
-    v.rhs = rhs;
     v.coef = G.dir[d].coef;
     v.ncell = G.dir[d].s + 2 * G.b + 1;
     v.uniform = G.dir[d].uniform ? 1 : 0;
@@ -1259,7 +1258,7 @@ int sweeps(const Fields &qin, const Fields &rhs, int rk, const Fields *qbase, co
             a.ci = ci;
             a.cdt = cdt;
         }
-        if (int rc = G.visc ? viscous(d, qin, rhs, a) : sweep(ld, a)) return rc;
+        if (int rc = G.visc ? viscous(d, qin, a) : sweep(ld, a)) return rc;
     }
     return 0;
 }

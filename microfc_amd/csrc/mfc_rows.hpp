@@ -94,7 +94,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
         if (fin_lane) {
             FinishIn<S> fin;
             finish_load<NF, D, FM>(a, go, ro, fin);
-            finish_cell<NF, D, double, FM, false>(a, go, ro, inv, fm, f, usm, us, fin, a.base_lo, a.base_hi, x, j, t);
+            finish_cell<NF, D, double, FM, false>(a, go, ro, inv, fm, f, usm, us, fin, a.base_lo, a.base_hi, x, j);
         }
     }
 }

@@ -332,26 +332,23 @@ __device__ __forceinline__ GhostSet ghosts_of(int i, int s, const int *bc, int b
     return e;
 }
 
-// Fills the ghost cells of the stage output that copy cell (i, j, k), whose
-// values are r: every combination of the cell's copies in each direction (the
-// reference's x, then y, then z fill), the momentum normal to a mirror
-// negated.  Saves a pass of k_bc_fill and its launch per RK stage after the
+// Fills the ghost cells of the stage output that copy cell (i, j), whose values
+// are r: every combination of the cell's copies in each direction (the
+// reference's x, then y fill), the momentum normal to a mirror negated.  Saves a pass of k_bc_fill and its launch per RK stage after the
 // first (RK3 step of 1000 cells: 30.0 -> 27.9 us; 768 x 768, contracted 188 ->
 // 176 us; 1024 x 1024 learned 514 -> 507 us).
 template <int NF, int D>
-__device__ __forceinline__ void store_ghosts(const SweepArgs &a, const SweepArgs &out, int i, int j, int k,
-                                             const double *r) {
+__device__ __forceinline__ void store_ghosts(const SweepArgs &a, const SweepArgs &out, int i, int j, const double *r) {
+    static_assert(D <= 2, "a 3D corner cell has 124 copies");
     using Y = Sys<NF, D>;
     constexpr int S = Y::S;
     if (!a.ghosts) return;
     bool edge = i < a.b || i > a.m - a.b;
     if constexpr (D > 1) edge = edge || j < a.b || j > a.n - a.b;
-    if constexpr (D > 2) edge = edge || k < a.b || k > a.p - a.b;
     if (!edge) return;
     const GhostSet none{0, 0, 0, 0, false, false};
     const GhostSet ex = ghosts_of(i, a.m, a.bcs[0], a.b);
     const GhostSet ey = D > 1 ? ghosts_of(j, a.n, a.bcs[1], a.b) : none;
-    const GhostSet ez = D > 2 ? ghosts_of(k, a.p, a.bcs[2], a.b) : none;
     // copy c of a direction: the cell itself, then the lower, then the upper
     // ghosts
     auto copy = [](const GhostSet &e, int c, int own, bool &flip) {
@@ -359,19 +356,16 @@ __device__ __forceinline__ void store_ghosts(const SweepArgs &a, const SweepArgs
         return c == 0 ? own : c <= e.n0 ? e.g0 + c - 1 : e.g1 + c - 1 - e.n0;
     };
 #pragma unroll 1
-    for (int ck = 0; ck <= ez.n0 + ez.n1; ++ck) {
+    for (int cj = 0; cj <= ey.n0 + ey.n1; ++cj) {
 #pragma unroll 1
-        for (int cj = 0; cj <= ey.n0 + ey.n1; ++cj) {
-#pragma unroll 1
-            for (int ci = cj == 0 && ck == 0 ? 1 : 0; ci <= ex.n0 + ex.n1; ++ci) {
-                bool f[3];
-                const int gi = copy(ex, ci, i, f[0]), gj = copy(ey, cj, j, f[1]), gk = copy(ez, ck, k, f[2]);
-                const long o = ghost_off(a, gi, gj, gk);
+        for (int ci = cj == 0 ? 1 : 0; ci <= ex.n0 + ex.n1; ++ci) {
+            bool f[2];
+            const int gi = copy(ex, ci, i, f[0]), gj = copy(ey, cj, j, f[1]);
+            const long o = ghost_off(a, gi, gj, 0);
 #pragma unroll
-                for (int v = 0; v < S; ++v) {
-                    const bool neg = v >= Y::MOM && v < Y::MOM + D && f[v - Y::MOM];
-                    out.qout.v[v][o] = neg ? -r[v] : r[v];
-                }
+            for (int v = 0; v < S; ++v) {
+                const bool neg = v >= Y::MOM && v < Y::MOM + D && f[v - Y::MOM];
+                out.qout.v[v][o] = neg ? -r[v] : r[v];
             }
         }
     }
@@ -415,7 +409,7 @@ __device__ __forceinline__ void rk_combine(const SweepArgs &a, const FinishIn<S>
 template <int NF, int D, typename R, int M, bool GH, typename O>
 __device__ __forceinline__ void finish_cell(const SweepArgs &a, O go, O ro, double inv,
                                             const R *Fm, const R *Fp, R usm, R usp,
-                                            const FinishIn<Sys<NF, D>::S> &f, int lo, int hi, int i, int j, int k) {
+                                            const FinishIn<Sys<NF, D>::S> &f, int lo, int hi, int i, int j) {
     using Y = Sys<NF, D>;
     constexpr int S = Y::S;
     double r[S];
@@ -458,7 +452,7 @@ __device__ __forceinline__ void finish_cell(const SweepArgs &a, O go, O ro, doub
             }
 #pragma unroll
             for (int v = 0; v < S; ++v) el(a.qout.v[v], go) = r[v];
-            if constexpr (GH) store_ghosts<NF, D>(a, a, i, j, k, r);
+            if constexpr (GH) store_ghosts<NF, D>(a, a, i, j, r);
             return;
         }
     }
@@ -489,7 +483,7 @@ __device__ __forceinline__ void finish_cell(const SweepArgs &a, O go, O ro, doub
             }
 #pragma unroll
             for (int v = 0; v < S; ++v) el(a.qout.v[v], go) = o[v];
-            if constexpr (GH) store_ghosts<NF, D>(a, a, i, j, k, o);
+            if constexpr (GH) store_ghosts<NF, D>(a, a, i, j, o);
             return;
         }
     }
@@ -866,7 +860,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(ML ? 2 : 4, 
             const Off go{ghost_off(a, x0, j, k), (unsigned)lane}, ro{interior_off(a, x0, j, k), (unsigned)lane};
             FinishIn<S> fin;
             finish_load_staged<NF, D, FM>(a, go, ro, cin, 1, fin);
-            finish_cell<NF, D, R, FM, GH>(a, go, ro, a.inv_ds[i], f, fp, us, usp, fin, a.base_lo, a.base_hi, i, j, k);
+            finish_cell<NF, D, R, FM, GH>(a, go, ro, a.inv_ds[i], f, fp, us, usp, fin, a.base_lo, a.base_hi, i, j);
         }
         return;
     }
@@ -903,7 +897,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(ML ? 2 : 4, 
         else
             finish_load<NF, D, FM>(a, go, ro, fin);
         finish_cell<NF, D, R, FM, GH>(a, go, ro, a.inv_ds[i], Fm, Fp, sf[S][lane], sf[S][lane + 1], fin,
-                                  a.base_lo, a.base_hi, i, j, k);
+                                  a.base_lo, a.base_hi, i, j);
     }
 }
 
@@ -1092,7 +1086,7 @@ __global__ __launch_bounds__(t_threads<ML>()) __attribute__((amdgpu_waves_per_eu
         else
             finish_load<NF, D, FM>(a, gcell(i, cc), rcell(i, cc), fin);
         finish_cell<NF, D, R, FM, false>(a, gcell(i, cc), rcell(i, cc), a.inv_ds[cc], Fm, Fp, sf[S][ts][tx],
-                                  sf[S][ts + 1][tx], fin, a.base_lo, a.base_hi, i, DIR == 1 ? cc : t, DIR == 1 ? t : cc);
+                                  sf[S][ts + 1][tx], fin, a.base_lo, a.base_hi, i, DIR == 1 ? cc : t);
     }
 }
 
@@ -1290,7 +1284,7 @@ __global__ __launch_bounds__((tc_cols<R, ML>(DIR) * tc_rows<R>(DIR)))
         else
             finish_load<NF, D, FM>(a, go, ro, fin);
         finish_cell<NF, D, R, FM, false>(a, go, ro, a.inv_ds[cc], Fm, Fp, fl[S][fs][fx], fl[S][fs + 1][fx], fin, a.base_lo,
-                                  a.base_hi, i, DIR == 1 ? cc : t, DIR == 1 ? t : cc);
+                                  a.base_hi, i, DIR == 1 ? cc : t);
     }
 }
 
@@ -1321,7 +1315,7 @@ __device__ __forceinline__ double finish_y_part(const SweepArgs &a, bool fold, d
 template <int NF, int D, typename R, bool GH, typename O, typename YP>
 __device__ __forceinline__ void finish_xy(const SweepArgs &a, const SweepArgs &out, O go, O ro, double ix, double iy,
                                           const double *dfx, double dusx, double dusy,
-                                          const FinishIn<Sys<NF, D>::S> &f, int i, int j, int k,
+                                          const FinishIn<Sys<NF, D>::S> &f, int i, int j,
                                           YP &&y_part) {
     using Y = Sys<NF, D>;
     constexpr int S = Y::S;
@@ -1347,7 +1341,7 @@ __device__ __forceinline__ void finish_xy(const SweepArgs &a, const SweepArgs &o
             rk_combine<S>(a, f, r, o);
 #pragma unroll
             for (int v = 0; v < S; ++v) el(out.qout.v[v], go) = o[v];
-            if constexpr (GH) store_ghosts<NF, D>(a, out, i, j, k, o);
+            if constexpr (GH) store_ghosts<NF, D>(a, out, i, j, o);
         }
         return;
     }
@@ -1370,7 +1364,7 @@ __device__ __forceinline__ void finish_xy(const SweepArgs &a, const SweepArgs &o
         }
 #pragma unroll
         for (int v = 0; v < S; ++v) el(out.qout.v[v], go) = r[v];
-        if constexpr (GH) store_ghosts<NF, D>(a, out, i, j, k, r);
+        if constexpr (GH) store_ghosts<NF, D>(a, out, i, j, r);
     } else {
 #pragma unroll
         for (int v = 0; v < S; ++v) r[v] = __builtin_fma(ix, dfx[v], y_part(v, false, iy));
@@ -1597,7 +1591,7 @@ __global__ __launch_bounds__(kXyThreads) __attribute__((amdgpu_waves_per_eu(4, 8
                 for (int v = 0; v < S; ++v) f.base[v] = a.base_is_in ? cin[v] : el(a.qbase.v[v], go);
             }
         }
-        finish_xy<NF, D, R, GH>(a, a, go, ro, ix, iy, dfx, dusx, dusy, f, i, j, k, [&](int v, bool fold, double sy) {
+        finish_xy<NF, D, R, GH>(a, a, go, ro, ix, iy, dfx, dusx, dusy, f, i, j, [&](int v, bool fold, double sy) {
             return finish_y_part<R>(
                 a, fold, sy, dfy[v], v >= a.base_lo && v < a.base_hi, [&] { return el(a.rhs.v[v], ro); },
                 [&] { return el(a.qbase.v[v], go); });

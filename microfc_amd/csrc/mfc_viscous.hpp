@@ -22,7 +22,6 @@ struct ViscParams {
 
 struct ViscArgs {
     Fields q;             // ghost-filled conservative stage input
-    Fields rhs;           // interior rhs the divergence is added to
     const double *coef;   // WENO coefficients of the sweep direction, 27 planes of ncell
     long ncell;
     int uniform;          // every reconstructed cell has the coefficients ucf (bit for bit)
