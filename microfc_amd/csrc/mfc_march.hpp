@@ -121,10 +121,13 @@ __device__ __forceinline__ void march_prim_in(const SweepArgs &a, const R *prim,
     }
 }
 
-// Waves per SIMD the kernel is compiled for.  FP64: two, with 154 to 254
+// Waves per SIMD the kernel is compiled for.  FP64: two, with 127 to 255
 // VGPRs and the next rows' loads a whole pass ahead.  At three (168 VGPRs) the
 // contracted x and y march spills 20 bytes, or takes its loads late: 512^3
-// 8.24 and 7.69 against 7.35 ms per launch.
+// 8.24 and 7.69 against 7.35 ms per launch.  On unequal widths, where a lane keeps
+// its cell's 27 x coefficients, the x and y march with two fluids spills even so:
+// plain 28 bytes of scratch per lane in 2D and 84 in 3D (92 with PO), FP32 bulk
+// 16 and 64 at its three waves.
 template <typename R>
 constexpr int march_waves() { return sizeof(R) == 4 ? 3 : 2; }
 

@@ -22,8 +22,8 @@ inline namespace MFC_FORM {
 // k_sweep_x reads the coefficients of both cells of a face per row, 54 loads
 // beside the S variables', and computes the smoothness indicators of each cell
 // twice, since a lane with one cell's both faces lost a wave of occupancy.
-// Here the loads are shared by the rows and two waves per SIMD are enough (161
-// to 232 VGPRs; at three the coefficients spill): 180 x 130 x 90 cells, three
+// Here the loads are shared by the rows and two waves per SIMD are enough (142
+// to 229 VGPRs; at three the coefficients spill): 180 x 130 x 90 cells, three
 // fluids, contracted 0.201 -> 0.151 ms per launch, 256 x 200 x 160 0.827 ->
 // 0.538, plain 700 x 700, two fluids 0.044 -> 0.037 ms.
 template <int NF, int D>

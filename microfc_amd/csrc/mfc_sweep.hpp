@@ -488,7 +488,9 @@ __device__ __forceinline__ void finish_cell(const SweepArgs &a, O go, O ro, doub
         }
     }
     // combined and stored per variable: with the results in an array first,
-    // k_sweep_t kept that array in scratch
+    // k_sweep_t kept that array in scratch, and with three fluids stored wrong
+    // partial densities (why was not found).  The kernels that have the array,
+    // above, keep none in scratch.
     switch (a.rk) {
     case kRkNone:
 #pragma unroll
