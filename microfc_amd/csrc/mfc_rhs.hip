@@ -46,17 +46,24 @@ constexpr long kPolls = 100000;
 // host code its name is not a device address; kernels get the address that
 // hipGetSymbolAddress returned for the current device (g_scratch_dev).
 static __device__ __align__(256) double scratch[kReduceBlocks];
+// Blocks of the running CFL reduction that are done (k_icfl, which leaves it 0).
+static __device__ unsigned icfl_done;
 
 namespace {
 
 // Held by the entry points that reduce over the cells, each until its value is
-// on the host: a case has one block counter and one result word (k_icfl), and
-// one array of partials for all but mfc_cfl_dt_noalloc.
+// on the host: they share one block counter per GPU and one result word
+// (k_icfl), and all but mfc_cfl_dt_noalloc the case's array of partials.
 std::mutex g_reduce;
+// The result word, pinned; made by the first mfc_rhs_init and held, as the
+// counter and `scratch` are, until the process ends (made per case, an init took
+// 244 instead of 202 us).
+double *g_result = nullptr;
 
-// Device address of `scratch` on each GPU, looked up once per device by
-// mfc_rhs_init with that device current.
+// Device addresses of `scratch` and `icfl_done` on each GPU, looked up once per
+// device by mfc_rhs_init with that device current.
 double *g_scratch_dev[kMaxDevices] = {};
+unsigned *g_done_dev[kMaxDevices] = {};
 
 constexpr int kNumFluidsBuilt = 10;   // the FP64 forms (every num_fluids the reference allows)
 constexpr int kNumFluidsBuiltF32 = 4; // the FP32-bulk and learned forms
@@ -169,8 +176,7 @@ struct State {
     hipStream_t own = nullptr, stream = nullptr;
     double *partials = nullptr; // 2 * kReduceBlocks doubles
     double *scratch = nullptr;  // this device's `scratch` array (kReduceBlocks doubles)
-    unsigned *count = nullptr;  // blocks of the running CFL reduction that are done (k_icfl)
-    double *result = nullptr;   // pinned: its value
+    unsigned *count = nullptr;  // this device's `icfl_done`
     double *scratch_state = nullptr; // S*ng doubles, RK3 stage buffer
     bool visc = false;               // any fluid_pp%Re > 0
     ViscParams vp{};
@@ -1303,10 +1309,7 @@ int mfc_rhs_init(const mfc_params *prm) {
     HIPCHK(hipStreamCreateWithFlags(&G.own, hipStreamNonBlocking));
     G.stream = G.own;
     HIPCHK(hipMalloc(&G.partials, sizeof(double) * 2 * kReduceBlocks));
-    HIPCHK(hipMalloc(&G.count, sizeof(unsigned)));
-    const unsigned none = 0;
-    HIPCHK(hipMemcpy(G.count, &none, sizeof none, hipMemcpyHostToDevice));
-    HIPCHK(hipHostMalloc(&G.result, sizeof(double), hipHostMallocDefault));
+    if (!g_result) HIPCHK(hipHostMalloc(&g_result, sizeof(double), hipHostMallocPortable));
     {
         int dev = 0;
         HIPCHK(hipGetDevice(&dev));
@@ -1315,8 +1318,11 @@ int mfc_rhs_init(const mfc_params *prm) {
             void *ptr = nullptr;
             HIPCHK(hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch)));
             g_scratch_dev[dev] = static_cast<double *>(ptr);
+            HIPCHK(hipGetSymbolAddress(&ptr, HIP_SYMBOL(icfl_done)));
+            g_done_dev[dev] = static_cast<unsigned *>(ptr);
         }
         G.scratch = g_scratch_dev[dev];
+        G.count = g_done_dev[dev];
     }
     // Re_size, Re_idx, Res (m_global_parameters.fpp:314-338, m_viscous.fpp:36-42)
     for (int r = 0; r < 2; ++r)
@@ -1367,10 +1373,13 @@ int mfc_rhs_set_grid(int dir, const double *s_cb, const double *ds) {
     // grid) keep cell -1's: with each cell's own, 1024^2 cells took 311 instead
     // of 234 us per step, 64^3 204 instead of 170.
     D.canon = D.uniform && G.prm.precision == MFC_PREC_FP64_FAST && G.prm.weno_order == 5;
-    for (int q = 0; q < kNCoef && D.canon; ++q)
-        for (int j = -1; j <= s + 1 && D.canon; ++j)
-            D.canon = std::fabs(D.coef_h[(long)q * (s + 2 * b + 1) + (j + b)] - kCanon[q]) <=
-                      kUniformRelTol * std::fabs(kCanon[q]);
+    for (int q = 0; q < kNCoef && D.canon; ++q) {
+        const double *c = &D.coef_h[(long)q * (s + 2 * b + 1) + (b - 1)], at = kCanon[q];
+        const double tol = kUniformRelTol * std::fabs(at);
+        int far = 0;
+        for (int j = 0; j < s + 3; ++j) far |= !(std::fabs(c[j] - at) <= tol);
+        D.canon = !far;
+    }
     // Uniform over every cell with coefficients (the weno_Re_flux gradient
     // pass reconstructs the ghost cells too)?
     {
@@ -1518,17 +1527,17 @@ static int icfl_reduce(double *const *q, bool from_cons, double dt, double *out,
     if (!partials || nb > capacity)
         return fail(-1, "CFL reduction needs %d partials, the buffer holds %d", nb, capacity);
     const hipStream_t st = G.stream;
-    *(volatile uint64_t *)G.result = kPending;
+    *(volatile uint64_t *)g_result = kPending;
     int rc;
     {
     TimedScope ts(timed ? kKIcfl : -1);
     rc = dispatch_nf_d([&](auto NF, auto D) -> int {
         if (from_cons)
             hipLaunchKernelGGL((k_icfl<decltype(NF)::value, decltype(D)::value, true>), dim3(nb), dim3(kCflThreads), 0,
-                               st, f, e, x, dxs[0], dxs[1], dxs[2], dt, G.nint, partials, G.count, G.result);
+                               st, f, e, x, dxs[0], dxs[1], dxs[2], dt, G.nint, partials, G.count, g_result);
         else
             hipLaunchKernelGGL((k_icfl<decltype(NF)::value, decltype(D)::value, false>), dim3(nb), dim3(kCflThreads), 0,
-                               st, f, e, x, dxs[0], dxs[1], dxs[2], dt, G.nint, partials, G.count, G.result);
+                               st, f, e, x, dxs[0], dxs[1], dxs[2], dt, G.nint, partials, G.count, g_result);
         HIPCHK(hipGetLastError());
         return 0;
     });
@@ -1539,10 +1548,10 @@ static int icfl_reduce(double *const *q, bool from_cons, double dt, double *out,
     // 18.2 us).  The kernels before it on the stream have then ended.  After
     // kPolls looks, a millisecond or two, the call waits for the stream, which
     // also reports errors.
-    volatile uint64_t *r = (volatile uint64_t *)G.result;
+    volatile uint64_t *r = (volatile uint64_t *)g_result;
     for (long n = 0; n < kPolls && *r == kPending; ++n) __builtin_ia32_pause();
     if (*r == kPending) HIPCHK(hipStreamSynchronize(st));
-    *out = *(volatile double *)G.result;
+    *out = *(volatile double *)g_result;
     return 0;
 }
 
@@ -1708,8 +1717,6 @@ int mfc_rhs_finalize(void) {
         G.dir[d] = Dir();
     }
     if (G.partials) (void)hipFree(G.partials);
-    if (G.count) (void)hipFree(G.count);
-    if (G.result) (void)hipHostFree(G.result);
     if (G.scratch_state) (void)hipFree(G.scratch_state);
     if (G.visc_grad) (void)hipFree(G.visc_grad);
     if (G.own) (void)hipStreamDestroy(G.own);
